@@ -508,7 +508,6 @@ int ocfd_create(const ocfd_config *cfg, int device, ocfd_handle **out) {
   if (cfg->scheme_invis == SCH_HYBRID) rc |= alloc(&B.rhyb, hb);
   if (cfg->if_viscous == 1) rc |= alloc(&B.ev, 12 * (size_t)B.g.ni * sizeof(double));
   if (cfg->nfiltering > 0) rc |= alloc(&h->fbuf, fb);
-  rc |= alloc(&B.trash, 16 * 256 * sizeof(double));
   for (int a = 0; a < 3; a++) {
     B.hlist[a] = B.hgbase[a] = nullptr;
     B.hbits[a] = nullptr;
@@ -585,7 +584,7 @@ int ocfd_destroy(ocfd_handle *h) {
   Block &B = h->B;
   for (const PrimField *p : {&B.d, &B.u, &B.v, &B.w, &B.T, &B.T2, &B.u2, &B.v2, &B.w2})
     if (p->p) (void)hipFree(p->p);
-  double *ps[] = {B.f, B.fn, B.du, B.rhyb, B.ev, B.trash, h->fbuf, h->work, h->wout};
+  double *ps[] = {B.f, B.fn, B.du, B.rhyb, B.ev, h->fbuf, h->work, h->wout};
   for (double *p : ps)
     if (p) (void)hipFree(p);
   for (int a = 0; a < 3; a++) {

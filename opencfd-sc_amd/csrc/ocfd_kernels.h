@@ -55,7 +55,6 @@ struct Block {
   double *f, *fn, *du;        // 5 planes each
   double *rhyb;               // halo'd sensor (hybrid scheme only)
   double *ev;                 // 12 interior planes: Ev1(1:4), Ev2(1:4), Ev3(1:4)
-  double *trash;              // 16 x 256 doubles: stores of lanes outside the block
   // hybrid scheme, per sweep axis: the faces that use WENO7/WENO5 (face id
   // * 2 + (WENO5)), their count, the face -> list slot map and the fluxes of
   // the listed faces (5 per face characteristic, 10 otherwise).  The map is
