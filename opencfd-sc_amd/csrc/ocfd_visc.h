@@ -12,9 +12,8 @@
 //               T <= 0 trap (whole-step path; du is not written back)
 //
 // k_visc_flux and k_visc_div_update march along k over a 64x4 tile of (i,j)
-// columns and a segment of up to 64 planes in FP64, 32 in FP32 (fewer on
-// small blocks so the launch still fills the chip).  The x and y neighbours of the current plane
-// come from a double-buffered LDS tile: while one plane is computed, every
+// columns and a segment of up to 64 planes in FP64, 32 in FP32 (march_kseg).
+// The x and y neighbours of the current plane come from a double-buffered LDS tile: while one plane is computed, every
 // lane already holds its share of the next plane's tile in registers, so
 // there is one barrier per plane and the loads overlap the arithmetic.  The
 // z neighbours of a lane's own column are a register queue of the 2R+1
@@ -561,17 +560,48 @@ __global__ __launch_bounds__(NT) void k_visc_div_update_batch(const BoxSet S, co
 // ---------------------------------------------------------------------------
 inline unsigned nblocks(int64_t n) { return (unsigned)((n + NT - 1) / NT); }
 
-// planes per workgroup: the longest segment that still gives about 2048
-// workgroups, at most 32 planes, for the FP32 kernels; about 1024 workgroups
-// of at most 64 planes for the FP64 ones, which run fewer waves per SIMD and
-// gain from amortising the prologue of their plane queue over a longer march
-template <typename RT>
-inline int march_kseg(const Geom &g) {
-  const int64_t cols = (int64_t)((g.nx + TXT - 1) / TXT) * ((g.ny + TYT - 1) / TYT);
-  const int64_t k = cols * g.nz / (sizeof(RT) == 8 ? 1024 : 2048);
-  const int kmax = sizeof(RT) == 8 ? KSEG_MAX : 32;
-  return (int)(k < 1 ? 1 : (k > kmax ? kmax : k));
+// workgroups of `kernel` (NT threads, static LDS) the device holds at once;
+// `cache` keeps the value per device for one kernel
+template <typename K>
+int resident_groups(K kernel, int (&cache)[64]) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (cache[dev] == 0) {
+    int cus = 0, per = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, NT, 0) != hipSuccess || per < 1) per = 1;
+    cache[dev] = cus * per;
+  }
+  return cache[dev];
 }
+
+// Planes per workgroup of a k-marching kernel: its time is close to the
+// number of rounds of resident workgroups times the planes of a segment plus
+// its prologue (the plane queue and the first tile, about 2.5 planes: 6.3 +
+// 2.45 us per plane of the FP64 update), so the length with the smallest
+// product is taken, the longer one at equal cost.  kmax: 64 in FP64, 32 in
+// FP32, measured best on large blocks, which any length near kmax serves.
+// A fixed count of workgroups instead gave 64^3 blocks one plane per
+// workgroup and left uneven last rounds: update of 101 x 75 x 54 FP64 51 us
+// against 38 now, 96^3 87 against 73, 128^3 CD8 145 against 134, 192^3 514
+// against 466, 160^3 with metric fields 334 against 304.
+inline int march_kseg(const Geom &g, int slots, int kmax) {
+  const int64_t cols = (int64_t)((g.nx + TXT - 1) / TXT) * ((g.ny + TYT - 1) / TYT);
+  if (kmax > g.nz) kmax = g.nz;
+  int best = kmax;
+  int64_t cost = INT64_MAX;
+  for (int k = kmax; k >= 1; k--) {
+    const int64_t groups = cols * ((g.nz + k - 1) / k);
+    const int64_t c = (groups + slots - 1) / slots * (2 * k + 5);
+    if (c < cost) {
+      cost = c;
+      best = k;
+    }
+  }
+  return best;
+}
+template <typename RT>
+constexpr int march_kmax() { return sizeof(RT) == 8 ? KSEG_MAX : 32; }
 inline unsigned march_blocks(const Geom &g, int kseg) {
   return (unsigned)(((g.nx + TXT - 1) / TXT) * ((g.ny + TYT - 1) / TYT) * ((g.nz + kseg - 1) / kseg));
 }
@@ -581,15 +611,19 @@ inline bool all_periodic(const Block &B) {
   return B.S.iperiodic[0] == 1 && B.S.iperiodic[1] == 1 && B.S.iperiodic[2] == 1 && B.M.uniform;
 }
 
+template <bool CD8, bool FAST, typename RT>
+void launch_flux_one(const Block &B, hipStream_t st) {
+  static int cache[64] = {};
+  const int kseg = march_kseg(B.g, resident_groups(k_visc_flux<CD8, FAST, RT>, cache), march_kmax<RT>());
+  hipLaunchKernelGGL((k_visc_flux<CD8, FAST, RT>), dim3(march_blocks(B.g, kseg)), dim3(NT), 0, st, B, kseg);
+}
 template <typename RT>
 hipError_t visc_flux_as(const Block &B, hipStream_t st) {
-  const int kseg = march_kseg<RT>(B.g);
-  const dim3 grid(march_blocks(B.g, kseg));
   const bool cd8 = B.S.scheme_vis == SCH_CD8, per = all_periodic(B);
-  if (cd8 && per) hipLaunchKernelGGL((k_visc_flux<true, true, RT>), grid, dim3(NT), 0, st, B, kseg);
-  else if (cd8) hipLaunchKernelGGL((k_visc_flux<true, false, RT>), grid, dim3(NT), 0, st, B, kseg);
-  else if (per) hipLaunchKernelGGL((k_visc_flux<false, true, RT>), grid, dim3(NT), 0, st, B, kseg);
-  else hipLaunchKernelGGL((k_visc_flux<false, false, RT>), grid, dim3(NT), 0, st, B, kseg);
+  if (cd8 && per) launch_flux_one<true, true, RT>(B, st);
+  else if (cd8) launch_flux_one<true, false, RT>(B, st);
+  else if (per) launch_flux_one<false, true, RT>(B, st);
+  else launch_flux_one<false, false, RT>(B, st);
   return hipGetLastError();
 }
 
@@ -599,19 +633,22 @@ hipError_t visc_div_as(const Block &B, hipStream_t st) {
   return hipGetLastError();
 }
 
+template <bool VISC, bool CD8, bool FAST, typename RT>
+void launch_update_one(const Block &B, int krk, int refresh_planes, int *neg, hipStream_t st) {
+  static int cache[64] = {};
+  const int kseg =
+      march_kseg(B.g, resident_groups(k_visc_div_update<VISC, CD8, FAST, RT>, cache), march_kmax<RT>());
+  hipLaunchKernelGGL((k_visc_div_update<VISC, CD8, FAST, RT>), dim3(march_blocks(B.g, kseg)), dim3(NT), 0, st, B, krk,
+                     refresh_planes, kseg, neg);
+}
 template <typename RT>
 hipError_t visc_div_update_as(const Block &B, int krk, int refresh_planes, int *neg, hipStream_t st) {
-  const int kseg = march_kseg<RT>(B.g);
-  const dim3 grid(march_blocks(B.g, kseg));
   const bool cd8 = B.S.scheme_vis == SCH_CD8, per = all_periodic(B);
-#define OCFD_DIVUPD(V, C, P) \
-  hipLaunchKernelGGL((k_visc_div_update<V, C, P, RT>), grid, dim3(NT), 0, st, B, krk, refresh_planes, kseg, neg)
-  if (B.ev == nullptr) OCFD_DIVUPD(false, false, false);
-  else if (cd8 && per) OCFD_DIVUPD(true, true, true);
-  else if (cd8) OCFD_DIVUPD(true, true, false);
-  else if (per) OCFD_DIVUPD(true, false, true);
-  else OCFD_DIVUPD(true, false, false);
-#undef OCFD_DIVUPD
+  if (B.ev == nullptr) launch_update_one<false, false, false, RT>(B, krk, refresh_planes, neg, st);
+  else if (cd8 && per) launch_update_one<true, true, true, RT>(B, krk, refresh_planes, neg, st);
+  else if (cd8) launch_update_one<true, true, false, RT>(B, krk, refresh_planes, neg, st);
+  else if (per) launch_update_one<true, false, true, RT>(B, krk, refresh_planes, neg, st);
+  else launch_update_one<true, false, false, RT>(B, krk, refresh_planes, neg, st);
   return hipGetLastError();
 }
 
