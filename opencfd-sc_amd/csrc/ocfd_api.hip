@@ -544,6 +544,7 @@ int ocfd_create(const ocfd_config *cfg, int device, ocfd_handle **out) {
     B.M.p[m] = h->met[m];
     B.M.u[m] = 1.0;
   }
+  set_split_const(B);
   // allocate_flow_data initial values (OCFD_NS_Solver.f90:116-118, 140-147)
   for (const PrimField *p : {&B.d, &B.u, &B.v, &B.w, &B.T, &B.T2}) (void)fill(*p, B.g.nh, 1.0, h->st);
   if (h->fused)
@@ -648,6 +649,7 @@ int ocfd_set_uniform_metrics(ocfd_handle *h, const double m[10]) {
   if (!h->B.M.uniform) return fail("ocfd_set_uniform_metrics needs OCFD_METRIC_UNIFORM");
   for (int q = 0; q < 10; q++) h->B.M.u[q] = m[q];
   for (int q = 0; q < 9; q++) h->B.M.u[M_AKX1 + q] = m[q] / m[M_AJAC];
+  set_split_const(h->B);
   invalidate_graph(h);  // the constants travel in the kernel arguments
   return 0;
 }

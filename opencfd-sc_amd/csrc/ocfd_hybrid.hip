@@ -109,7 +109,7 @@ void k_weno_faces(const Block B) {
   const SchemeParams &S = B.S;
   const int n = g.n(AXIS);
   const int tid = threadIdx.x;
-  const double gamma = B.P.gamma, rma = B.P.ma;
+  const double gamma = B.P.gamma;
   const int q1 = M_AKX1 + 3 * AXIS;
   const int count = B.hcount[AXIS];
   const int nbatch = (count + FB - 1) / FB;
@@ -165,10 +165,8 @@ void k_weno_faces(const Block B) {
           const int fb = it >> 3, p = it & 7;
           const double dd = pv[r][0], uu = pv[r][1], vv = pv[r][2], ww = pv[r][3], Tt = pv[r][4];
           const double A1 = B.M.u[q1], A2 = B.M.u[q1 + 1], A3 = B.M.u[q1 + 2];
-          SplitK<RR> K;
-          split_k_gamma(RR(gamma), K);
-          split_k_metric(RR(A1), RR(A2), RR(A3), sw, K);
-          const RR ccr = sqrt(RR(Tt)) / RR(rma);
+          const SplitK<RR> &K = split_const<RR>(B, AXIS);
+          const RR ccr = div_known(RR(sqrt(RR(Tt))), K.ma, K.rma);
           RR fp[5], fm[5];
           if (sw) split_sw<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);
           else split_llf<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);
@@ -179,7 +177,7 @@ void k_weno_faces(const Block B) {
           }
           if (CHAR && (p == 3 || p == 4)) {
             double *q = sQ[fb][p - 3];
-            q[0] = uu; q[1] = vv; q[2] = ww; q[3] = sqrt(Tt) / rma;
+            q[0] = uu; q[1] = vv; q[2] = ww; q[3] = div_known(sqrt(Tt), B.sk64[AXIS].ma, B.sk64[AXIS].rma);
             q[4] = A1; q[5] = A2; q[6] = A3;
           }
         }
@@ -193,16 +191,13 @@ void k_weno_faces(const Block B) {
       TI::face_of(g, list[f0 + fb] >> 1, s, w, c);
       const int64_t h = TI::hidx(g, s - 3 + p, w, c);
       const double dd = B.d[h], uu = B.u[h], vv = B.v[h], ww = B.w[h], Tt = B.T[h];
-      const double cc = sqrt(Tt) / rma;
+      const double cc = div_known(sqrt(Tt), B.sk64[AXIS].ma, B.sk64[AXIS].rma);
       const double A1 = (FAST || B.M.uniform) ? B.M.u[q1] : B.M.p[q1][h];
       const double A2 = (FAST || B.M.uniform) ? B.M.u[q1 + 1] : B.M.p[q1 + 1][h];
       const double A3 = (FAST || B.M.uniform) ? B.M.u[q1 + 2] : B.M.p[q1 + 2][h];
-      // the splitting's constants per point (held across the batch loop they
-      // would cost registers, i.e. occupancy)
-      SplitK<RR> K;
-      split_k_gamma(RR(gamma), K);
-      split_k_metric(RR(A1), RR(A2), RR(A3), sw, K);
-      const RR ccr = sqrt(RR(Tt)) / RR(rma);  // OCFD_inviscous.f90:67, in the splitting's type
+      SplitK<RR> K = split_const<RR>(B, AXIS);
+      if (!FAST && !B.M.uniform) split_k_metric(RR(A1), RR(A2), RR(A3), sw, K);
+      const RR ccr = div_known(RR(sqrt(RR(Tt))), K.ma, K.rma);  // OCFD_inviscous.f90:67, in the splitting's type
       RR fp[5], fm[5];
       if (sw) split_sw<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);
       else split_llf<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);

@@ -38,6 +38,8 @@ struct Block {
   SchemeParams S;
   Phys P;
   Metrics M;
+  SplitK<double> sk64[3];     // constants of the flux splittings per sweep axis
+  SplitK<float> sk32[3];
   PrimField d, u, v, w, T;    // halo'd primitives
   // The temperature the stage being computed writes.  comput_duvwT repairs a
   // cell with T <= 0 from its six neighbours in the reference's i-j-k loop,
@@ -74,6 +76,23 @@ struct Block {
   // nothing, so the state stays that of the failing stage.
   int *halt;
 };
+template <typename R>
+__device__ inline const SplitK<R> &split_const(const Block &B, int axis) {
+  if constexpr (sizeof(R) == 8) return B.sk64[axis];
+  else return B.sk32[axis];
+}
+// fills sk64, sk32 from the block's parameters and, on a uniform grid, its
+// metrics: after any change of either
+inline void set_split_const(Block &B) {
+  const bool sw = B.S.flux_split == 1;
+  for (int a = 0; a < 3; a++) {
+    const double *A = &B.M.u[M_AKX1 + 3 * a];
+    split_k_gamma(B.P.gamma, B.P.ma, B.sk64[a]);
+    split_k_metric(A[0], A[1], A[2], sw, B.sk64[a]);
+    split_k_gamma(float(B.P.gamma), float(B.P.ma), B.sk32[a]);
+    split_k_metric(float(A[0]), float(A[1]), float(A[2]), sw, B.sk32[a]);
+  }
+}
 // the kernels of a precision read the primitives in their real type: FP32
 // fields belong to the mixed-precision form, FP64 fields to the FP64 path
 inline bool prims_match(const Block &B) {

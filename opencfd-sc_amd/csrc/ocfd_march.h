@@ -46,12 +46,8 @@ __device__ __forceinline__ void march_line(const Block &B, const int i, const in
   const R *const pd = B.d.as<R>(), *const pu = B.u.as<R>(), *const pv = B.v.as<R>(), *const pw = B.w.as<R>(),
           *const pT = B.T.as<R>();
   R *const du = reinterpret_cast<R *>(B.du);
-  const int q1 = M_AKX1 + 3 * AXIS;
   const bool sw = S.flux_split == 1;
-  SplitK<R> K;
-  split_k_gamma(R(B.P.gamma), K);
-  split_k_metric(R(B.M.u[q1]), R(B.M.u[q1 + 1]), R(B.M.u[q1 + 2]), sw, K);
-  const R rma = R(B.P.ma);
+  const SplitK<R> K = split_const<R>(B, AXIS);
   const R hinv = R(B.P.hinv[AXIS]);
   const R ajac = R(B.M.u[M_AJAC]);
   const int64_t hstep = g.hstride(AXIS), istep = g.istride(AXIS);
@@ -100,7 +96,7 @@ __device__ __forceinline__ void march_line(const Block &B, const int i, const in
       // ---- split fluxes of point s0 - 4 + pi, then the loads PD points ahead ----
       {
         const R dd = pr[slot][0], uu = pr[slot][1], vv = pr[slot][2], ww = pr[slot][3];
-        const R cc = sqrt(pr[slot][4]) / rma;  // OCFD_inviscous.f90:67
+        const R cc = div_known(R(sqrt(pr[slot][4])), K.ma, K.rma);  // OCFD_inviscous.f90:67
         if (sw) split_sw<R>(K, cc, dd, uu, vv, ww, qp[j], qm[j]);
         else split_llf<R>(K, cc, dd, uu, vv, ww, qp[j], qm[j]);
       }

@@ -36,10 +36,11 @@ __device__ constexpr inline int lidx(int m, int p, int wl) {
   return AXIS == 0 ? (m * TW + wl) * NPT + p : (m * NPT + p) * TW + wl;
 }
 
-// One tile b of a sweep of block B.  FAST: the sweep axis is periodic (no
+// One tile b of a sweep of block B.  FAST != 0: the sweep axis is periodic (no
 // block-edge closures) and the metrics are uniform, both known at compile
-// time.
-template <int AXIS, int SCH, bool CHAR, int TL, int TW, bool FAST, typename R>
+// time; 2: the metric vector of the axis also points along its own
+// coordinate (axis_aligned), which the projecting schemes make use of.
+template <int AXIS, int SCH, bool CHAR, int TL, int TW, int FAST, typename R>
 __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode) {
   typedef TileIndex<AXIS> TI;
   constexpr int NP = TL + 8;  // points s0-4 .. s0+TL+3
@@ -47,7 +48,7 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   constexpr bool HYB = (SCH == SCH_HYBRID);
   constexpr int NH = CHAR ? 5 : 10;
   constexpr int NI1 = (NP * TW + NTHREADS - 1) / NTHREADS;      // points per thread
-  constexpr int NI3 = (5 * TL * TW + NTHREADS - 1) / NTHREADS;  // du entries per thread
+  static_assert(TL * TW == NTHREADS, "one cell of the tile per thread in phase 3");
   // characteristic inputs per point: u, v, w, c (+ the three normalised
   // metrics when they vary in space)
   const bool unif = FAST || B.M.uniform != 0;
@@ -63,7 +64,7 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   const int c = b / ntw + 1;
   const int s0 = 1 + ts * TL, w0 = 1 + tw * TW;
   const int tid = threadIdx.x;
-  const double gamma = B.P.gamma, rma = B.P.ma;
+  const double gamma = B.P.gamma;
   const int q1 = M_AKX1 + 3 * AXIS;
   const SchemeParams &S = B.S;
   const int lo = S.bidx[AXIS][0], hi = S.bidx[AXIS][1];
@@ -75,13 +76,9 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
     if (AXIS == 0) { p = it % NP; wl = it / NP; } else { wl = it % TW; p = it / TW; }
     return it < NP * TW && s0 - 4 + p <= n + LAP && w0 + wl <= nw;
   };
-  // du entry handled by phase-3 slot r
-  auto p3 = [&](int r, int &sl_, int &wl, int &m) {
-    const int it = tid + r * NTHREADS;
-    if (AXIS == 0) { sl_ = it % TL; wl = (it / TL) % TW; m = it / (TL * TW); }
-    else { wl = it % TW; sl_ = (it / TW) % TL; m = it / (TL * TW); }
-    return it < 5 * TL * TW && s0 + sl_ <= n && w0 + wl <= nw;
-  };
+  // the cell (five du entries) of this thread in phase 3
+  const int c3s = AXIS == 0 ? tid % TL : tid / TW, c3w = AXIS == 0 ? tid / TL : tid % TW;
+  const bool c3 = s0 + c3s <= n && w0 + c3w <= nw;
 
   // primitives of the tile's points (stored in the sweep's real type)
   R pq[NI1][5];
@@ -104,7 +101,8 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   // fluxes are computed
   // du is stored in the sweep's real type (FP32 in the mixed-precision form)
   R *const du = reinterpret_cast<R *>(B.du);
-  R pdu[NI3];
+  R pdu[5];
+  const int64_t c3i = TI::iidx(g, s0 + c3s, w0 + c3w, c);
 
   R *sF = reinterpret_cast<R *>(smem);             // fp(5), fm(5)      [10][NP][TW]
   // the characteristic inputs are needed only where the sweep itself
@@ -121,18 +119,14 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   R *sH = ALIAS ? sF : sQend;                      // face fluxes       [NH][NF][TW]
   int *sS = reinterpret_cast<int *>(ALIAS ? sQend : sH + NH * NF * TW);  // hybrid: list slot of each face [NF][TW]
   // ---- phase 1: split fluxes at the tile's points ----
-  // the splitting's constants once per thread (and the metric part once per
-  // sweep on a uniform grid)
   const bool sw = S.flux_split == 1;
-  SplitK<R> K;
-  split_k_gamma(R(gamma), K);
-  if (unif) split_k_metric(R(B.M.u[q1]), R(B.M.u[q1 + 1]), R(B.M.u[q1 + 2]), sw, K);
+  SplitK<R> K = split_const<R>(B, AXIS);
 #pragma unroll
   for (int r = 0; r < NI1; r++) {
     int p, wl;
     if (!p1(r, p, wl)) continue;
     const R dd = R(pq[r][0]), uu = R(pq[r][1]), vv = R(pq[r][2]), ww = R(pq[r][3]);
-    const R cc = sqrt(R(pq[r][4])) / R(rma);  // OCFD_inviscous.f90:67
+    const R cc = div_known(sqrt(R(pq[r][4])), K.ma, K.rma);  // OCFD_inviscous.f90:67
     if (!unif) {
       const int64_t h = TI::hidx(g, s0 - 4 + p, w0 + wl, c);
       split_k_metric(R(B.M.p[q1][h]), R(B.M.p[q1 + 1][h]), R(B.M.p[q1 + 2][h]), sw, K);
@@ -182,29 +176,37 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   }
   __syncthreads();
 
-  if (mode != INV_ASSIGN) {
+  if (mode != INV_ASSIGN && c3) {
 #pragma unroll
-    for (int r = 0; r < NI3; r++) {
-      int sl_, wl, m;
-      if (!p3(r, sl_, wl, m)) continue;
-      pdu[r] = du[TI::iidx(g, s0 + sl_, w0 + wl, c) + (int64_t)m * g.ni];
-    }
+    for (int m = 0; m < 5; m++) pdu[m] = du[c3i + (int64_t)m * g.ni];
   }
 
   // ---- phase 2: face fluxes ----
+  // strides of a point and of a component in the split-flux array: a face's
+  // stencil is read as constant offsets from one address (each value's own
+  // index cost 40 integer instructions per 16 reads)
+  constexpr int PS = AXIS == 0 ? 1 : TW, CS = NP * TW;
   // flux+/- of component m at face f (non-characteristic)
   auto face_nc = [&](int m, int f, int wl, int s, int scm, R &hp, R &hm) {
     R xp[8], xm[8];
+    const R *const q = sF + lidx<AXIS, NP, TW>(m, f, wl);
 #pragma unroll
     for (int k = 0; k < 8; k++) {
-      xp[k] = sF[lidx<AXIS, NP, TW>(m, f + k, wl)];
-      xm[k] = sF[lidx<AXIS, NP, TW>(5 + m, f + k, wl)];
+      xp[k] = q[k * PS];
+      xm[k] = q[5 * CS + k * PS];
     }
     hp = FAST ? inner_p<SCH>(S, xp, scm) : face_p_nonchar<SCH>(S, xp, s, n, AXIS, scm);
     hm = FAST ? inner_m<SCH>(S, xm, scm) : face_m_nonchar<SCH>(S, xm, s, n, AXIS, scm);
   };
-#define FPV(m, k) sF[lidx<AXIS, NP, TW>((m), f + (k), wl)]
-#define FMV(m, k) sF[lidx<AXIS, NP, TW>(5 + (m), f + (k), wl)]
+  // (fs: the face's first stencil point)
+// after a characteristic row: the next one reads its stencil again (kept in
+// registers across the rows, the 80 values took half the occupancy)
+#define ROW_END                          \
+  asm volatile("" ::: "memory");         \
+  __builtin_amdgcn_sched_barrier(0)
+#define FACE_STENCIL const R *const fs = sF + lidx<AXIS, NP, TW>(0, f, wl)
+#define FPV(m, k) fs[(m) * CS + (k) * PS]
+#define FMV(m, k) fs[(5 + (m)) * CS + (k) * PS]
   // all five components of face f, projected on the characteristic basis of
   // the face unless the face is linear (flux_charteric,
   // OCFD_inviscous_character.f90:190-290)
@@ -228,45 +230,47 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
 #undef QV
     char_basis<R>(R(gamma), u1, v1, w1, c1, a1, a2, a3, Bs);
   };
+  // The projected stencil values x(k) = sum over components c of S(r,c) *
+  // f(c,k), lo <= k <= hi, 0 elsewhere, of flux + (p = 0) or flux - (p = 5),
+  // summed in the reference's order c = 1..5.  One flux is projected and
+  // reconstructed before the other, and the empty asm keeps each component's
+  // products before the next one's loads: with both fluxes or all 40 stencil
+  // values in flight a WENO7 row takes up to 60 more registers, and the tiles
+  // lose a wave or two per SIMD.
+  // (stencils: set_parameters, OCFD_readpara.f90:261-341)
+  constexpr int a1h = SCH == SCH_WENO5 ? -2 : -3, b1h = SCH == SCH_WENO5 ? 2 : (SCH == SCH_WENO7 ? 3 : 4);
+  constexpr int a2h = SCH == SCH_WENO5 ? -1 : (SCH == SCH_WENO7 ? -2 : -3), b2h = SCH == SCH_WENO5 ? 3 : 4;
+  auto project = [&](int f, int wl, int p, const R *sr5, R *x, const int lo, const int hi) {
+    FACE_STENCIL;
+#pragma unroll
+    for (int k = 0; k < 8; k++) x[k] = k >= lo && k <= hi ? sr5[0] * FPV(p, k) : R(0.0);
+#pragma unroll
+    for (int c = 1; c < 5; c++) {
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (k >= lo && k <= hi) asm volatile("" : "+v"(x[k]) : : "memory");
+#pragma unroll
+      for (int k = 0; k < 8; k++)
+        if (k >= lo && k <= hi) x[k] = madd(sr5[c], FPV(p + c, k), x[k]);
+    }
+  };
   // characteristic flux h0(r) = h+(r) + h-(r) of face f: row r of S applied
   // to the split fluxes on the scheme's stencil, then reconstructed
   // (OCFD_inviscous_character.f90:250-282)
   auto char_row = [&](const CharBasisT<R> &Bs, int f, int wl, int s, int scm, int r) {
-    int a1h = S.ka1, b1h = S.kb1, a2h = S.ka2, b2h = S.kb2;
-    if (HYB) {
-      if (scm == 2) { a1h = -3; b1h = 3; a2h = -2; b2h = 4; }
-      else if (scm == 3) { a1h = -2; b1h = 2; a2h = -1; b2h = 3; }
-    }
-    R xp[8], xm[8], sr5[5];
+    R x[8], sr5[5];
     char_S_row(Bs, r, sr5);
-    // xp(k) = sum over components c of S(r,c) * fp(c,k), summed in the
-    // reference's order c = 1..5; outside the scheme's stencil the value is 0
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      xp[k] = sr5[0] * FPV(0, k);
-      xm[k] = sr5[0] * FMV(0, k);
-    }
-#pragma unroll
-    for (int c = 1; c < 5; c++) {
-      // keeps the scheduler from fetching all 80 stencil values at once
-      __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-      for (int k = 0; k < 8; k++) {
-        xp[k] = madd(sr5[c], FPV(c, k), xp[k]);
-        xm[k] = madd(sr5[c], FMV(c, k), xm[k]);
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-      if (k < a1h + 3 || k > b1h + 3) xp[k] = R(0.0);
-      if (k < a2h + 3 || k > b2h + 3) xm[k] = R(0.0);
-    }
-    const R h1 = FAST ? inner_p<SCH>(S, xp, scm) : face_p_char<SCH>(S, xp, s, n, AXIS, scm);
-    const R h2 = FAST ? inner_m<SCH>(S, xm, scm) : face_m_char<SCH>(S, xm, s, n, AXIS, scm);
+    // outside the scheme's stencil the projected value is 0
+    project(f, wl, 0, sr5, x, a1h + 3, b1h + 3);
+    const R h1 = FAST ? inner_p<SCH>(S, x, scm) : face_p_char<SCH>(S, x, s, n, AXIS, scm);
+    __builtin_amdgcn_sched_barrier(0);
+    project(f, wl, 5, sr5, x, a2h + 3, b2h + 3);
+    const R h2 = FAST ? inner_m<SCH>(S, x, scm) : face_m_char<SCH>(S, x, s, n, AXIS, scm);
     return h1 + h2;
   };
   // component m of a linear (hybrid UD7L) face: no projection
   auto linear_comp = [&](int f, int wl, int s, int m) {
+    FACE_STENCIL;
     R xp[8], xm[8];
 #pragma unroll
     for (int k = 0; k < 8; k++) { xp[k] = FPV(m, k); xm[k] = FMV(m, k); }
@@ -277,22 +281,115 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   // non-reflecting closure of component m (OCFD_inviscous_character.f90:295-309);
   // point t is k = t - s + 3
   auto closure_comp = [&](int f, int wl, int s, int m) {
+    FACE_STENCIL;
     if (s == 0)
       return (R(2.0) * FPV(m, 4) + R(5.0) * FPV(m, 5) - FPV(m, 6) + R(2.0) * FMV(m, 6) - R(7.0) * FMV(m, 5) +
               R(11.0) * FMV(m, 4)) / R(6.0);
     return (R(2.0) * FPV(m, 1) - R(7.0) * FPV(m, 2) + R(11.0) * FPV(m, 3) + R(2.0) * FMV(m, 3) +
             R(5.0) * FMV(m, 2) - FMV(m, 1)) / R(6.0);
   };
+  // The same for a metric vector along the sweep's own coordinate: the face
+  // normal and the two tangents are unit vectors, so the basis needs no
+  // square root and no division but those of c, and the two rows of the
+  // tangential velocities have two entries (-u_t and +-1) instead of five.
+  // The terms left out are products with an exact 0 or 1, the order of the
+  // others stays, so finite fluxes are the same bits.  The projection of
+  // two rows and 96 of 400 LDS reads per face go, and the rows' code is
+  // straight-line (the loop of face_ch indexes its row at run time).  WENO7
+  // sweeps of 192^3: FP64 835-857 us with the general form, 650-710 with this
+  // one; FP32 330-355 and 270-293.
+  auto face_aligned = [&](int f, int wl, R *hh) {
+    FACE_STENCIL;
+    constexpr int IL = AXIS == 0 ? 1 : 0, IM = AXIS == 2 ? 1 : 2;  // the tangents' coordinates
+    constexpr int SL = AXIS == 0 ? 1 : -1, SM = AXIS == 2 ? -1 : 1;  // and signs
+    R v[3], c1;
+    {
+#define QV(q, k) sQ[lidx<AXIS, NP, TW>((q), f + (k), wl)]
+#pragma unroll
+      for (int q = 0; q < 3; q++) v[q] = (QV(q, 3) + QV(q, 4)) * R(0.5);
+      c1 = (QV(3, 3) + QV(3, 4)) * R(0.5);
+#undef QV
+    }
+    const R un = v[AXIS], ul = SL > 0 ? v[IL] : -v[IL], um = SM > 0 ? v[IM] : -v[IM];
+    const R V2 = (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) * R(0.5);
+    const R KK = (R(gamma) - R(1.0)) / (c1 * c1);
+    const R KK1 = KK * R(0.5);
+    const R X1 = R(1.0) / (R(2.0) * c1);
+    const R H = V2 + R(1.0) / KK;
+    auto dense = [&](const R *sr5) {
+      R x[8];
+      project(f, wl, 0, sr5, x, a1h + 3, b1h + 3);
+      const R hp = inner_p<SCH>(S, x, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      project(f, wl, 5, sr5, x, a2h + 3, b2h + 3);
+      return hp + inner_m<SCH>(S, x, 0);
+    };
+    auto sparse = [&](R s0, int q, int sign) {
+      R x[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        x[k] = s0 * FPV(0, k);
+        x[k] = sign > 0 ? x[k] + FPV(q, k) : x[k] - FPV(q, k);
+      }
+      const R hp = inner_p<SCH>(S, x, 0);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int k = 0; k < 8; k++) {
+        x[k] = s0 * FMV(0, k);
+        x[k] = sign > 0 ? x[k] + FMV(q, k) : x[k] - FMV(q, k);
+      }
+      return hp + inner_m<SCH>(S, x, 0);
+    };
+    R h0[5], sr5[5];
+    sr5[0] = R(1.0) - KK * V2;
+#pragma unroll
+    for (int q = 0; q < 3; q++) sr5[1 + q] = KK * v[q];
+    sr5[4] = -KK;
+    h0[0] = dense(sr5);
+    ROW_END;
+    h0[1] = sparse(-ul, 1 + IL, SL);
+    ROW_END;
+    h0[2] = sparse(-um, 1 + IM, SM);
+    ROW_END;
+    sr5[0] = KK1 * V2 + X1 * un;
+#pragma unroll
+    for (int q = 0; q < 3; q++) sr5[1 + q] = q == AXIS ? -X1 - KK1 * v[q] : -(KK1 * v[q]);
+    sr5[4] = KK1;
+    h0[3] = dense(sr5);
+    ROW_END;
+    sr5[0] = KK1 * V2 - X1 * un;
+    sr5[1 + AXIS] = X1 - KK1 * v[AXIS];
+    h0[4] = dense(sr5);
+    ROW_END;
+    hh[0] = h0[0] + h0[3] + h0[4];
+#pragma unroll
+    for (int q = 0; q < 3; q++) {
+      R a = v[q] * h0[0];
+      if (q == IL) a = SL > 0 ? a + h0[1] : a - h0[1];
+      if (q == IM) a = SM > 0 ? a + h0[2] : a - h0[2];
+      a = madd(q == AXIS ? v[q] - c1 : v[q], h0[3], a);
+      hh[1 + q] = madd(q == AXIS ? v[q] + c1 : v[q], h0[4], a);
+    }
+    const R a = madd(um, h0[2], madd(ul, h0[1], V2 * h0[0]));
+    hh[4] = madd(madd(c1, un, H), h0[4], madd(madd(-c1, un, H), h0[3], a));
+  };
   // all five components of face f, projected on the characteristic basis of
   // the face (flux_charteric, OCFD_inviscous_character.f90:190-290)
   auto face_ch = [&](int f, int wl, int s, int scm, R *hh) {
+    if constexpr (FAST == 2) {
+      face_aligned(f, wl, hh);
+      return;
+    }
     CharBasisT<R> Bs;
     basis_of(f, wl, Bs);
     R h0[5];
     // one row at a time: unrolled, the five rows' stencils stayed live
     // together (FP32 tiles at 256 VGPRs plus AGPRs, one wave per SIMD)
 #pragma unroll 1
-    for (int r = 0; r < 5; r++) h0[r] = char_row(Bs, f, wl, s, scm, r);
+    for (int r = 0; r < 5; r++) {
+      h0[r] = char_row(Bs, f, wl, s, scm, r);
+      ROW_END;
+    }
     char_back(Bs, h0, hh);
   };
   auto listed = [&](int f, int wl) { return sS[lidx<AXIS, NF, TW>(0, f, wl)] >= 0; };
@@ -325,11 +422,17 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   // one tail item: face FULL + tid / 5, component / row tid % 5; stage 1 of
   // a projected face leaves its row in sTail, stage 2 (after a barrier)
   // returns the component
-  auto tail_row = [&](CharBasisT<R> &Bs, int f, int wl, int s, int row) {
+  // (the basis is formed again in stage 2: kept across the row's projection
+  // its 21 values set the kernel's register count, 194 against 126 for WENO7
+  // in FP64)
+  auto tail_row = [&](int f, int wl, int s, int row) {
+    CharBasisT<R> Bs;
     basis_of(f, wl, Bs);
     sTail[tid] = char_row(Bs, f, wl, s, 0, row);
   };
-  auto tail_back = [&](const CharBasisT<R> &Bs, int row) {
+  auto tail_back = [&](int f, int wl, int row) {
+    CharBasisT<R> Bs;
+    basis_of(f, wl, Bs);
     R h0[5], hh[5];
 #pragma unroll
     for (int q = 0; q < 5; q++) h0[q] = sTail[(tid / 5) * 5 + q];
@@ -373,10 +476,9 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
           const bool act = decode(r, m, f, wl);
           const int s = s0 - 1 + f;
           const bool clo = (closure_lo && s == 0) || (closure_hi && s == n);
-          CharBasisT<R> Bs;
-          if (act && !clo) tail_row(Bs, f, wl, s, m);
+          if (act && !clo) tail_row(f, wl, s, m);
           __syncthreads();
-          if (act) hv[r][0] = clo ? closure_comp(f, wl, s, m) : tail_back(Bs, m);
+          if (act) hv[r][0] = clo ? closure_comp(f, wl, s, m) : tail_back(f, wl, m);
           continue;
         }
       }
@@ -461,10 +563,9 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
         const bool act = decode(NI2 - 1, m, f, wl);
         const int s = s0 - 1 + f;
         const bool clo = (closure_lo && s == 0) || (closure_hi && s == n);
-        CharBasisT<R> Bs;
-        if (act && !clo) tail_row(Bs, f, wl, s, m);
+        if (act && !clo) tail_row(f, wl, s, m);
         __syncthreads();
-        if (act) sH[lidx<AXIS, NF, TW>(m, f, wl)] = clo ? closure_comp(f, wl, s, m) : tail_back(Bs, m);
+        if (act) sH[lidx<AXIS, NF, TW>(m, f, wl)] = clo ? closure_comp(f, wl, s, m) : tail_back(f, wl, m);
       }
     } else {
       // hybrid, characteristic: the linear and closure faces, all five
@@ -506,44 +607,44 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   }
 #undef FPV
 #undef FMV
+#undef FACE_STENCIL
+#undef ROW_END
   __syncthreads();
 
   // ---- phase 3: flux difference into du ----
+  if (!c3) return;
   const double hinv = B.P.hinv[AXIS];
+  const R *const hf = sH + lidx<AXIS, NF, TW>(0, c3s, c3w);  // face s - 1 of the cell; face s is PS further
+  constexpr int HS = NF * TW;
 #pragma unroll
-  for (int r = 0; r < NI3; r++) {
-    int sl_, wl, m;
-    if (!p3(r, sl_, wl, m)) continue;
-    const int s = s0 + sl_, w = w0 + wl;
-    const int f = sl_ + 1;
+  for (int m = 0; m < 5; m++) {
     R val;
     if (!CHAR) {
-      val = (sH[lidx<AXIS, NF, TW>(m, f, wl)] - sH[lidx<AXIS, NF, TW>(m, f - 1, wl)] +
-             sH[lidx<AXIS, NF, TW>(5 + m, f, wl)] - sH[lidx<AXIS, NF, TW>(5 + m, f - 1, wl)]) * R(hinv);
+      val = (hf[m * HS + PS] - hf[m * HS] + hf[(5 + m) * HS + PS] - hf[(5 + m) * HS]) * R(hinv);
     } else {
-      val = (sH[lidx<AXIS, NF, TW>(m, f, wl)] - sH[lidx<AXIS, NF, TW>(m, f - 1, wl)]) * R(hinv);
+      val = (hf[m * HS + PS] - hf[m * HS]) * R(hinv);
     }
-    const int64_t q = TI::iidx(g, s, w, c) + (int64_t)m * g.ni;
+    R *const dst = du + c3i + (int64_t)m * g.ni;
     if (mode == INV_ASSIGN) {
-      du[q] = val;
+      *dst = val;
     } else if (mode == INV_ACCUM) {
-      du[q] = pdu[r] + val;
+      *dst = pdu[m] + val;
     } else {
-      const int64_t h = TI::hidx(g, s, w, c);
-      R rr = -(pdu[r] + val) * R(FAST ? B.M.u[M_AJAC] : B.M.get(M_AJAC, h));
+      const int64_t h = TI::hidx(g, s0 + c3s, w0 + c3w, c);
+      R rr = -(pdu[m] + val) * R(FAST ? B.M.u[M_AJAC] : B.M.get(M_AJAC, h));
       if (B.P.if_mass_force == 1 && m > 0) {
         // OCFD_inviscous.f90:189-201
         const double *mf = B.P.mass_force;
         if (m < 4) rr = rr + R(B.d[h] * mf[m - 1]);
         else rr = rr + R(B.d[h] * (B.u[h] * mf[0] + B.v[h] * mf[1] + B.w[h] * mf[2]));
       }
-      du[q] = rr;
+      *dst = rr;
     }
   }
 }
 
 // one block: the tiles in XCD order
-template <int AXIS, int SCH, bool CHAR, int TL, int TW, bool FAST, typename R>
+template <int AXIS, int SCH, bool CHAR, int TL, int TW, int FAST, typename R>
 __global__ __launch_bounds__(NTHREADS) void k_inviscid(const Block B, const int mode) {
   sweep_tile<AXIS, SCH, CHAR, TL, TW, FAST, R>(B, xcd_tile(blockIdx.x, gridDim.x), mode);
 }
@@ -556,7 +657,7 @@ __global__ __launch_bounds__(NTHREADS) void k_inviscid_batch(const BoxSet S, con
   const int j = S.entry(t);
   // the descriptor is read in place (a local copy would live in scratch:
   // the sweep indexes some of its arrays at run time)
-  sweep_tile<AXIS, SCH, CHAR, TL, TW, true, R>(S.blk[S.ids[j]], t - S.off[j], mode);
+  sweep_tile<AXIS, SCH, CHAR, TL, TW, 1, R>(S.blk[S.ids[j]], t - S.off[j], mode);
 }
 
 // LDS bytes of a sweep tile: split fluxes, characteristic inputs, face fluxes
@@ -568,7 +669,7 @@ constexpr size_t sweep_lds(int nq) {
          (HYB ? sizeof(int) * (TL + 1) * TW : 0);
 }
 
-template <int AXIS, int SCH, bool CHAR, int TL, int TW, bool FAST, typename R>
+template <int AXIS, int SCH, bool CHAR, int TL, int TW, int FAST, typename R>
 hipError_t launch_one(const Block &B, int mode, hipStream_t st) {
   constexpr bool HYB = (SCH == SCH_HYBRID);
   static_assert(sweep_lds<TL, TW, CHAR, HYB, R>(7) <= 64 * 1024, "tile too large for LDS");
@@ -592,7 +693,7 @@ constexpr int shape_tl(int shape) {
   return AXIS == 0 ? (shape == 1 ? 32 : (shape == 2 ? 128 : 64)) : (shape == 1 ? 16 : (shape == 2 ? 64 : 32));
 }
 
-template <int AXIS, bool CHAR, bool FAST, typename R, int SHAPE>
+template <int AXIS, bool CHAR, int FAST, typename R, int SHAPE>
 hipError_t dispatch_scheme(const Block &B, int mode, hipStream_t st) {
   constexpr int TL = shape_tl<AXIS>(SHAPE);
   constexpr int TW = NTHREADS / TL;
@@ -601,7 +702,8 @@ hipError_t dispatch_scheme(const Block &B, int mode, hipStream_t st) {
     case SCH_WENO7: return launch_one<AXIS, SCH_WENO7, CHAR, TL, TW, FAST, R>(B, mode, st);
     case SCH_OMP6: return launch_one<AXIS, SCH_OMP6, CHAR, TL, TW, FAST, R>(B, mode, st);
     case SCH_UD7L: return launch_one<AXIS, SCH_UD7L, CHAR, TL, TW, FAST, R>(B, mode, st);
-    case SCH_HYBRID: return launch_one<AXIS, SCH_HYBRID, CHAR, TL, TW, FAST, R>(B, mode, st);
+    // (its faces are not projected in the sweep)
+    case SCH_HYBRID: return launch_one<AXIS, SCH_HYBRID, CHAR, TL, TW, FAST ? 1 : 0, R>(B, mode, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -631,6 +733,15 @@ hipError_t dispatch_march(const Block &B, int mode, int shape, hipStream_t st) {
   }
 }
 
+// whether a uniform grid's metric vector of the axis points along its own
+// coordinate, in the positive direction (every uniform box that is not
+// rotated or skewed)
+template <int AXIS>
+bool axis_aligned(const Metrics &M) {
+  const double *A = &M.u[M_AKX1 + 3 * AXIS];
+  return A[AXIS] > 0.0 && A[(AXIS + 1) % 3] == 0.0 && A[(AXIS + 2) % 3] == 0.0;
+}
+
 template <int AXIS, typename R>
 hipError_t dispatch_axis(const Block &B, int mode, int shape, hipStream_t st) {
   const bool ch = B.S.is_char != 0;
@@ -639,17 +750,17 @@ hipError_t dispatch_axis(const Block &B, int mode, int shape, hipStream_t st) {
   if (fast) {
     if (shape >= 3)
       return ch ? dispatch_march<AXIS, true, R>(B, mode, shape, st) : dispatch_march<AXIS, false, R>(B, mode, shape, st);
+    // a projecting sweep with a metric vector askew of its coordinate has the
+    // default tile only
+    if (ch && B.S.scheme_invis != SCH_HYBRID && !axis_aligned<AXIS>(B.M))
+      return dispatch_scheme<AXIS, true, 1, R, 0>(B, mode, st);
     if (shape == 1)
-      return ch ? dispatch_scheme<AXIS, true, true, R, 1>(B, mode, st)
-                : dispatch_scheme<AXIS, false, true, R, 1>(B, mode, st);
+      return ch ? dispatch_scheme<AXIS, true, 2, R, 1>(B, mode, st) : dispatch_scheme<AXIS, false, 1, R, 1>(B, mode, st);
     if (shape == 2)
-      return ch ? dispatch_scheme<AXIS, true, true, R, 2>(B, mode, st)
-                : dispatch_scheme<AXIS, false, true, R, 2>(B, mode, st);
-    return ch ? dispatch_scheme<AXIS, true, true, R, 0>(B, mode, st)
-              : dispatch_scheme<AXIS, false, true, R, 0>(B, mode, st);
+      return ch ? dispatch_scheme<AXIS, true, 2, R, 2>(B, mode, st) : dispatch_scheme<AXIS, false, 1, R, 2>(B, mode, st);
+    return ch ? dispatch_scheme<AXIS, true, 2, R, 0>(B, mode, st) : dispatch_scheme<AXIS, false, 1, R, 0>(B, mode, st);
   }
-  return ch ? dispatch_scheme<AXIS, true, false, R, 0>(B, mode, st)
-            : dispatch_scheme<AXIS, false, false, R, 0>(B, mode, st);
+  return ch ? dispatch_scheme<AXIS, true, 0, R, 0>(B, mode, st) : dispatch_scheme<AXIS, false, 0, R, 0>(B, mode, st);
 }
 
 // the three axes of one real type; shape selects the tile (periodic
