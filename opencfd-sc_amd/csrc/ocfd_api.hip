@@ -365,8 +365,7 @@ int inviscid(ocfd_handle *h, bool ch) {
     // hybrid: the WENO faces of the three sweeps first
     if ((h->cfg.if_scheme_character != 0) != ch)
       return fail("hybrid scheme: the inviscid routine must match IF_Scheme_Character");
-    for (int a = 0; a < 3; a++)
-      if (launch(h, "weno_faces", [&] { return launch_weno_faces(B, a, h->st); })) return -1;
+    if (launch(h, "weno_faces", [&] { return launch_weno_faces(B, h->st); })) return -1;
   }
   static const char *nm[2][3] = {{"inviscid_x", "inviscid_y", "inviscid_z"},
                                  {"inviscid_char_x", "inviscid_char_y", "inviscid_char_z"}};

@@ -686,6 +686,24 @@ __device__ inline void char_back(const CharBasisT<T> &B, const T *h0, T *hh) {
   hh[4] = row(B.V2, B.ul, B.um, B.H, B.un);
 }
 
+// row m of S1: S1 * h0 is madd(s[4], h0[4], ... madd(s[1], h0[1], s[0] * h0[0])),
+// the operations of char_back
+template <typename T>
+__device__ inline void char_S1_row(const CharBasisT<T> &B, int m, T *s) {
+  auto pick = [m](T x, T y, T z, T e) { return m == 1 ? x : (m == 2 ? y : (m == 3 ? z : e)); };
+  if (m == 0) {
+    s[0] = s[3] = s[4] = T(1.0);
+    s[1] = s[2] = T(0.0);
+    return;
+  }
+  const T nq = pick(B.n1, B.n2, B.n3, B.un), q = pick(B.u1, B.v1, B.w1, B.H);
+  s[0] = pick(B.u1, B.v1, B.w1, B.V2);
+  s[1] = pick(B.l1, B.l2, B.l3, B.ul);
+  s[2] = pick(B.m1, B.m2, B.m3, B.um);
+  s[3] = madd(-B.c1, nq, q);
+  s[4] = madd(B.c1, nq, q);
+}
+
 // ---------------------------------------------------------------------------
 // central first derivative of a field along an axis at interior point s of n
 // (OCFD_dx0/dy0/dz0, OCFD_dxyz_viscous.f90:3-239).  `o(d)` returns the field

@@ -8,10 +8,11 @@
 //   k_hyb_list    listed once per step, per sweep axis (a range of the
 //                 list reserved per workgroup, faces in order inside it),
 //                 with a face -> slot map for the sweeps;
-//   k_weno_faces  computed densely before each stage's sweeps: batches of
-//                 listed faces per workgroup, split fluxes of the 8 stencil
-//                 points in LDS, then one (face, characteristic row) -- or
-//                 (face, component) without projection -- per lane.
+//   k_weno_faces  computed densely before each stage's sweeps: batches of 64
+//                 listed faces on five wavefronts each, split fluxes of the 8
+//                 stencil points in LDS, then one characteristic row -- or
+//                 component, without projection -- per wavefront, one face
+//                 per lane.
 // The sweep kernels read the listed faces' fluxes by slot.  Every flux is the
 // same expression as in the sweep (flux_charteric,
 // OCFD_inviscous_character.f90:190-290; OCFD2d_flux1/2,
@@ -22,9 +23,9 @@ namespace ocfd {
 
 namespace {
 
-constexpr int FB = 51;   // listed faces per workgroup batch: 5 * FB rows fill the 256 lanes
-constexpr int SFS = 81;  // LDS stride of one face's split fluxes (8 points x 10, padded so
-                         // that the faces a wavefront reads fall in different banks)
+constexpr int FB = 64;           // listed faces of a batch: one per lane
+constexpr int NSUB = 3;          // batches a workgroup works on together
+constexpr int WNT = NSUB * 5 * FB;  // per batch a wavefront for each characteristic row / component
 
 // A workgroup lists LPT * NT consecutive faces of the axis: scheme index from
 // the sensor, the WENO faces appended to the axis list in face order, and the
@@ -91,279 +92,320 @@ __global__ __launch_bounds__(NT) void k_hyb_list(const Block B) {
   }
 }
 
-// Fluxes of the listed faces of one axis.  A fixed grid strides over batches
-// of FB faces; the list length is read from the device counter.  RR is the
-// real type of the splitting and the WENO reconstruction: double, or float
+// Fluxes of the listed faces of one axis: workgroup wg of nwg strides over
+// batches of FB faces; the list length is read from the device counter.  RR is
+// the real type of the splitting and the WENO reconstruction: double, or float
 // in the mixed-precision form, where the characteristic basis and the
-// projections onto and back from it stay FP64.
-template <int AXIS, bool CHAR, bool FAST, typename RR>
-__global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(sizeof(RR) == 4 ? 4 : 1)))
-void k_weno_faces(const Block B) {
+// projections onto and back from it stay FP64.  MET as in the sweeps: 0
+// closures and metric fields, 1 periodic axis and uniform metrics, 2 also a
+// metric vector along the axis' own coordinate.
+//
+// Of the five wavefronts of a batch, wavefront r works on row (component) r
+// of its 64 faces, so the row is the same for all its lanes: its entries of
+// the basis are formed by scalar branches, and with MET 2 the two rows of the
+// tangential velocities project two components instead of five.  The split
+// fluxes lie [component][point][face]: every LDS access is 64 consecutive
+// values.  Wavefront r also splits stencil points r and r + 5.  While a batch
+// is projected and reconstructed, the primitives of the next one and the list
+// entries of the one after are in flight (two dependent loads, about as long
+// as the arithmetic of a batch), and a lane keeps its face's coefficients in
+// registers to the end: two barriers per batch.  A workgroup takes three
+// batches at once: as workgroups of five wavefronts only two fitted a CU (the
+// first SIMD takes two of each five), 2.1 wavefronts per SIMD instead of 3.7.
+// Bound by instruction issue (VALU 65% busy).  256^3, 5.7% of the faces, three
+// axes: FP64 780 us in the former layout (256 lanes on 51 faces, one lane per
+// row: every lane formed all rows' entries, three launches), 695 with five
+// wavefronts per workgroup, 557 now; mixed (8.3%) 705, 550, 541; 160^3 FP64
+// with metric fields (8.6%) 414, 372, 323.
+template <int AXIS, bool CHAR, int MET, typename RR>
+__device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, double *const sQa, double *const sGa,
+                                                const int wg, const int nwg) {
   typedef TileIndex<AXIS> TI;
   constexpr int NH = CHAR ? 5 : 10;
-  __shared__ RR sF[FB][SFS];        // fp(1:5), fm(1:5) at stencil points s-3 .. s+4: [p * 10 + m]
-  __shared__ double sQ[FB][2][7];   // u, v, w, c, A1..A3 at points s, s+1
-  __shared__ double sB[FB][21];     // characteristic basis of the face
-  __shared__ double sG[FB][5];      // characteristic fluxes h0(1:5)
   const Geom &g = B.g;
   const SchemeParams &S = B.S;
   const int n = g.n(AXIS);
-  const int tid = threadIdx.x;
-  const double gamma = B.P.gamma;
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int sub = wave / 5, row = wave - 5 * sub;
+  RR *const sF = sFa + sub * (80 * FB);
+  double *const sQ = sQa + sub * (CHAR ? 14 * FB : 0), *const sG = sGa + sub * (CHAR ? 5 * FB : 0);
   const int q1 = M_AKX1 + 3 * AXIS;
   const int count = B.hcount[AXIS];
-  const int nbatch = (count + FB - 1) / FB;
-  const int *list = B.hlist[AXIS];
-  double *out = B.wflux[AXIS];
+  const int ngroup = (count + NSUB * FB - 1) / (NSUB * FB);  // groups of NSUB batches
+  const int *const list = B.hlist[AXIS];
+  double *const out = B.wflux[AXIS];
   const bool sw = S.flux_split == 1;
-  // batches in one contiguous range per XCD (workgroup b runs on XCD
+  const bool unif = MET != 0 || B.M.uniform != 0;
+  // groups in one contiguous range per XCD (workgroup b runs on XCD
   // b % NXCD), strided over that XCD's workgroups: list-neighbouring faces,
   // whose y / z stencils share rows, then meet in the same L2
-  const int nw = (int)gridDim.x / NXCD, xcd = (int)blockIdx.x % NXCD;
-  const bool split = (int)gridDim.x % NXCD == 0 && nw > 0;
-  const int blo = split ? (int)((int64_t)nbatch * xcd / NXCD) : 0;
-  const int bhi = split ? (int)((int64_t)nbatch * (xcd + 1) / NXCD) : nbatch;
-  const int b0 = split ? blo + (int)blockIdx.x / NXCD : (int)blockIdx.x;
-  const int bstep = split ? nw : (int)gridDim.x;
-  // The FP32 form with uniform metrics loads the primitives of its next
-  // batch's stencil points right after splitting the current batch's, so the
-  // loads run during the current batch's projection and reconstruction (the
-  // FP64 form has no registers to spare for them).
-  constexpr bool PF = FAST && sizeof(RR) == 4;
-  constexpr int NPI = (8 * FB + NT - 1) / NT;  // stencil points per lane and batch
-  float pv[PF ? NPI : 1][5];
-  auto fetch = [&](int bt) {
-    const int fn0 = bt * FB;
-    const int nfn = count - fn0 < FB ? count - fn0 : FB;
-#pragma unroll
-    for (int r = 0; r < NPI; r++) {
-      const int it = tid + r * NT;
-      if (bt < bhi && it < nfn * 8) {
-        const int fb = it >> 3, p = it & 7;
-        int s, w, c;
-        TI::face_of(g, list[fn0 + fb] >> 1, s, w, c);
-        const int64_t h = TI::hidx(g, s - 3 + p, w, c);
-        pv[r][0] = B.d.template as<float>()[h];
-        pv[r][1] = B.u.template as<float>()[h];
-        pv[r][2] = B.v.template as<float>()[h];
-        pv[r][3] = B.w.template as<float>()[h];
-        pv[r][4] = B.T.template as<float>()[h];
-      }
-    }
+  const int nw = nwg / NXCD, xcd = wg % NXCD;
+  const bool split = nwg % NXCD == 0 && nw > 0;
+  const int bhi = split ? (int)((int64_t)ngroup * (xcd + 1) / NXCD) : ngroup;
+  const int b0 = split ? (int)((int64_t)ngroup * xcd / NXCD) + wg / NXCD : wg;
+  const int bstep = split ? nw : nwg;
+  if (b0 >= bhi) return;
+  const RR *const P[5] = {B.d.as<RR>(), B.u.as<RR>(), B.v.as<RR>(), B.w.as<RR>(), B.T.as<RR>()};
+  // entry of this lane in group bt (past the end: the last one again)
+  auto entry = [&](int bt) {
+    const int f = (bt * NSUB + sub) * FB + lane;
+    return list[f < count ? f : count - 1];
   };
-  if constexpr (PF) fetch(b0);
-  for (int batch = b0; batch < bhi; batch += bstep) {
-    const int f0 = batch * FB;
-    const int nf = count - f0 < FB ? count - f0 : FB;
-    if constexpr (PF) {
-      // split fluxes at the stencil points from the prefetched primitives
-      // (the same values the loop below reads: FP32 storage, widened)
+  // stencil points row and row + 5 (< 8) of this lane's face
+  RR pv[2][5];
+  auto fetch = [&](int code) {
+    int s, w, c;
+    TI::face_of(g, code >> 1, s, w, c);
+    const int64_t h0 = TI::hidx(g, s - 3, w, c), st = g.hstride(AXIS);
 #pragma unroll
-      for (int r = 0; r < NPI; r++) {
-        const int it = tid + r * NT;
-        if (it < nf * 8) {
-          const int fb = it >> 3, p = it & 7;
-          const double dd = pv[r][0], uu = pv[r][1], vv = pv[r][2], ww = pv[r][3], Tt = pv[r][4];
-          const double A1 = B.M.u[q1], A2 = B.M.u[q1 + 1], A3 = B.M.u[q1 + 2];
-          const SplitK<RR> &K = split_const<RR>(B, AXIS);
-          const RR ccr = div_known(RR(sqrt(RR(Tt))), K.ma, K.rma);
-          RR fp[5], fm[5];
-          if (sw) split_sw<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);
-          else split_llf<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);
+    for (int r = 0; r < 2; r++)
+      if (row + 5 * r < 8) {
+        const int64_t h = h0 + (row + 5 * r) * st;
 #pragma unroll
-          for (int m = 0; m < 5; m++) {
-            sF[fb][p * 10 + m] = fp[m];
-            sF[fb][p * 10 + 5 + m] = fm[m];
-          }
-          if (CHAR && (p == 3 || p == 4)) {
-            double *q = sQ[fb][p - 3];
-            q[0] = uu; q[1] = vv; q[2] = ww; q[3] = div_known(sqrt(Tt), B.sk64[AXIS].ma, B.sk64[AXIS].rma);
-            q[4] = A1; q[5] = A2; q[6] = A3;
-          }
-        }
+        for (int q = 0; q < 5; q++) pv[r][q] = P[q][h];
       }
-      fetch(batch + bstep);
-    }
+  };
+  int code = entry(b0);
+  fetch(code);
+  int code1 = entry(b0 + bstep < bhi ? b0 + bstep : b0);
+  for (int batch = b0; batch < bhi; batch += bstep) {
+    int s, w, c;
+    TI::face_of(g, code >> 1, s, w, c);
     // split fluxes at the stencil points (OCFD_inviscous.f90:64-70, split_*)
-    for (int it = tid; !PF && it < nf * 8; it += NT) {
-      const int fb = it >> 3, p = it & 7;
-      int s, w, c;
-      TI::face_of(g, list[f0 + fb] >> 1, s, w, c);
-      const int64_t h = TI::hidx(g, s - 3 + p, w, c);
-      const double dd = B.d[h], uu = B.u[h], vv = B.v[h], ww = B.w[h], Tt = B.T[h];
-      const double cc = div_known(sqrt(Tt), B.sk64[AXIS].ma, B.sk64[AXIS].rma);
-      const double A1 = (FAST || B.M.uniform) ? B.M.u[q1] : B.M.p[q1][h];
-      const double A2 = (FAST || B.M.uniform) ? B.M.u[q1 + 1] : B.M.p[q1 + 1][h];
-      const double A3 = (FAST || B.M.uniform) ? B.M.u[q1 + 2] : B.M.p[q1 + 2][h];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+      const int p = row + 5 * r;
+      if (p >= 8) continue;
+      const RR dd = pv[r][0], uu = pv[r][1], vv = pv[r][2], ww = pv[r][3], Tt = pv[r][4];
       SplitK<RR> K = split_const<RR>(B, AXIS);
-      if (!FAST && !B.M.uniform) split_k_metric(RR(A1), RR(A2), RR(A3), sw, K);
-      const RR ccr = div_known(RR(sqrt(RR(Tt))), K.ma, K.rma);  // OCFD_inviscous.f90:67, in the splitting's type
+      double A[3] = {0.0, 0.0, 0.0};
+      if (!unif) {
+        const int64_t h = TI::hidx(g, s - 3 + p, w, c);
+#pragma unroll
+        for (int q = 0; q < 3; q++) A[q] = B.M.p[q1 + q][h];
+        split_k_metric(RR(A[0]), RR(A[1]), RR(A[2]), sw, K);
+      }
+      const RR ccr = div_known(RR(sqrt(Tt)), K.ma, K.rma);  // OCFD_inviscous.f90:67, in the splitting's type
       RR fp[5], fm[5];
-      if (sw) split_sw<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);
-      else split_llf<RR>(K, ccr, RR(dd), RR(uu), RR(vv), RR(ww), fp, fm);
+      if (sw) split_sw<RR>(K, ccr, dd, uu, vv, ww, fp, fm);
+      else split_llf<RR>(K, ccr, dd, uu, vv, ww, fp, fm);
 #pragma unroll
       for (int m = 0; m < 5; m++) {
-        sF[fb][p * 10 + m] = fp[m];
-        sF[fb][p * 10 + 5 + m] = fm[m];
+        sF[(m * 8 + p) * FB + lane] = fp[m];
+        sF[((5 + m) * 8 + p) * FB + lane] = fm[m];
       }
       if (CHAR && (p == 3 || p == 4)) {
-        double *q = sQ[fb][p - 3];
-        q[0] = uu; q[1] = vv; q[2] = ww; q[3] = cc;
-        q[4] = A1; q[5] = A2; q[6] = A3;
+        double *const q = sQ + (p - 3) * 7 * FB + lane;
+        q[0 * FB] = uu;
+        q[1 * FB] = vv;
+        q[2 * FB] = ww;
+        q[3 * FB] = div_known(sqrt(double(Tt)), B.sk64[AXIS].ma, B.sk64[AXIS].rma);
+        if (!unif) {
+#pragma unroll
+          for (int a = 0; a < 3; a++) q[(4 + a) * FB] = A[a];
+        }
       }
+    }
+    const int f = (batch * NSUB + sub) * FB + lane;
+    const int scm = (code & 1) ? 3 : 2;
+    code = code1;
+    if (batch + bstep < bhi) {
+      fetch(code);
+      code1 = entry(batch + 2 * bstep < bhi ? batch + 2 * bstep : batch + bstep);
     }
     __syncthreads();
-    if (CHAR) {
-      // basis from the face-averaged state (OCFD_inviscous_character.f90:200-236)
-      for (int fb = tid; fb < nf; fb += NT) {
-        const double *qa = sQ[fb][0], *qb = sQ[fb][1];
-        const double u1 = (qa[0] + qb[0]) * 0.5, v1 = (qa[1] + qb[1]) * 0.5;
-        const double w1 = (qa[2] + qb[2]) * 0.5, c1 = (qa[3] + qb[3]) * 0.5;
-        const double a1 = (qa[4] + qb[4]) * 0.5, a2 = (qa[5] + qb[5]) * 0.5, a3 = (qa[6] + qb[6]) * 0.5;
-        CharBasis Bs;
-        char_basis(gamma, u1, v1, w1, c1, a1, a2, a3, Bs);
-        double *o = sB[fb];
-        o[0] = Bs.u1; o[1] = Bs.v1; o[2] = Bs.w1; o[3] = Bs.c1; o[4] = Bs.n1; o[5] = Bs.n2; o[6] = Bs.n3;
-        o[7] = Bs.l1; o[8] = Bs.l2; o[9] = Bs.l3; o[10] = Bs.m1; o[11] = Bs.m2; o[12] = Bs.m3;
-        o[13] = Bs.un; o[14] = Bs.ul; o[15] = Bs.um; o[16] = Bs.V2; o[17] = Bs.KK; o[18] = Bs.KK1;
-        o[19] = Bs.X1; o[20] = Bs.H;
+    const RR *const F = sF + lane;
+    auto recon_p = [&](const RR *x) {
+      if (!CHAR) return MET ? inner_p<SCH_HYBRID>(S, x, scm) : face_p_nonchar<SCH_HYBRID>(S, x, s, n, AXIS, scm);
+      return MET ? inner_p<SCH_HYBRID>(S, x, scm) : face_p_char<SCH_HYBRID>(S, x, s, n, AXIS, scm);
+    };
+    auto recon_m = [&](const RR *x) {
+      if (!CHAR) return MET ? inner_m<SCH_HYBRID>(S, x, scm) : face_m_nonchar<SCH_HYBRID>(S, x, s, n, AXIS, scm);
+      return MET ? inner_m<SCH_HYBRID>(S, x, scm) : face_m_char<SCH_HYBRID>(S, x, s, n, AXIS, scm);
+    };
+    if constexpr (!CHAR) {
+      // flux+ and flux- of component `row`
+      RR x[8];
+#pragma unroll
+      for (int k = 0; k < 8; k++) x[k] = F[(row * 8 + k) * FB];
+      const double hp = recon_p(x);
+#pragma unroll
+      for (int k = 0; k < 8; k++) x[k] = F[((5 + row) * 8 + k) * FB];
+      const double hm = recon_m(x);
+      if (f < count) {
+        out[(int64_t)f * NH + row] = hp;
+        out[(int64_t)f * NH + 5 + row] = hm;
       }
-      __syncthreads();
-      auto basis = [&](int fb) {
-        const double *o = sB[fb];
-        CharBasis Bs;
-        Bs.u1 = o[0]; Bs.v1 = o[1]; Bs.w1 = o[2]; Bs.c1 = o[3]; Bs.n1 = o[4]; Bs.n2 = o[5]; Bs.n3 = o[6];
-        Bs.l1 = o[7]; Bs.l2 = o[8]; Bs.l3 = o[9]; Bs.m1 = o[10]; Bs.m2 = o[11]; Bs.m3 = o[12];
-        Bs.un = o[13]; Bs.ul = o[14]; Bs.um = o[15]; Bs.V2 = o[16]; Bs.KK = o[17]; Bs.KK1 = o[18];
-        Bs.X1 = o[19]; Bs.H = o[20];
-        return Bs;
-      };
-      // one characteristic row per lane: project, reconstruct (flux_x1/x2)
-      for (int it = tid; it < nf * 5; it += NT) {
-        const int fb = it / 5, r = it - 5 * fb;
-        const int code = list[f0 + fb];
-        const int scm = (code & 1) ? 3 : 2;
-        int s, w, c;
-        TI::face_of(g, code >> 1, s, w, c);
-        const CharBasis Bs = basis(fb);
-        double sr5[5];
-        char_S_row(Bs, r, sr5);
-        // stencils of the hybrid's WENO7 / WENO5 faces (Ka1_H2.. / Ka1_H3..)
-        const int a1h = scm == 2 ? -3 : -2, b1h = scm == 2 ? 3 : 2;
-        const int a2h = scm == 2 ? -2 : -1, b2h = scm == 2 ? 4 : 3;
-        // projection in FP64, reconstruction in RR
-        double xp[8], xm[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-          xp[k] = sr5[0] * double(sF[fb][k * 10]);
-          xm[k] = sr5[0] * double(sF[fb][k * 10 + 5]);
-        }
-        // (FP64 path: the reference's two roundings; the mixed form's FP64
-        // projection fuses them)
-        auto acc = [](double a, double b, double c) { return sizeof(RR) == 8 ? madd(a, b, c) : fma(a, b, c); };
-#pragma unroll
-        for (int cmp = 1; cmp < 5; cmp++) {
-#pragma unroll
-          for (int k = 0; k < 8; k++) {
-            xp[k] = acc(sr5[cmp], double(sF[fb][k * 10 + cmp]), xp[k]);
-            xm[k] = acc(sr5[cmp], double(sF[fb][k * 10 + 5 + cmp]), xm[k]);
-          }
-        }
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-          if (k < a1h + 3 || k > b1h + 3) xp[k] = 0.0;
-          if (k < a2h + 3 || k > b2h + 3) xm[k] = 0.0;
-        }
-        auto recon = [&](const auto *yp, const auto *ym) {
-          const auto h1 = FAST ? inner_p<SCH_HYBRID>(S, yp, scm) : face_p_char<SCH_HYBRID>(S, yp, s, n, AXIS, scm);
-          const auto h2 = FAST ? inner_m<SCH_HYBRID>(S, ym, scm) : face_m_char<SCH_HYBRID>(S, ym, s, n, AXIS, scm);
-          return double(h1 + h2);
-        };
-        if constexpr (sizeof(RR) == 8) {
-          sG[fb][r] = recon(xp, xm);
-        } else {
-          RR yp[8], ym[8];
-#pragma unroll
-          for (int k = 0; k < 8; k++) {
-            yp[k] = RR(xp[k]);
-            ym[k] = RR(xm[k]);
-          }
-          sG[fb][r] = recon(yp, ym);
-        }
-      }
-      __syncthreads();
-      // back to conservative components (S1 * h0): one (face, component)
-      // per lane, so the stores of a wavefront are contiguous
-      for (int it = tid; it < nf * 5; it += NT) {
-        const int fb = it / 5, m = it - 5 * fb;
-        const CharBasis Bs = basis(fb);
-        double hh[5];
-        char_back(Bs, sG[fb], hh);
-        out[(int64_t)(f0 + fb) * NH + m] = hh[m];
-      }
+      __syncthreads();  // the next batch overwrites the split fluxes
     } else {
-      // one component per lane: flux+ and flux- of the face
-      for (int it = tid; it < nf * 5; it += NT) {
-        const int fb = it / 5, m = it - 5 * fb;
-        const int code = list[f0 + fb];
-        const int scm = (code & 1) ? 3 : 2;
-        int s, w, c;
-        TI::face_of(g, code >> 1, s, w, c);
-        RR xp[8], xm[8];
+      // basis from the face-averaged state (OCFD_inviscous_character.f90:200-236)
+      double a[7];
+#pragma unroll
+      for (int q = 0; q < 7; q++) {
+        if (q < 4 || !unif) a[q] = (sQ[q * FB + lane] + sQ[(7 + q) * FB + lane]) * 0.5;
+        else a[q] = (B.M.u[q1 + q - 4] + B.M.u[q1 + q - 4]) * 0.5;
+      }
+      const double gamma = B.P.gamma;
+      // row `row` of S (with MET 2 rows 1 and 2 are sr5[0] and sg at component
+      // tq) and of S1; a product with an exact 0 or 1 changes no finite sum
+      double sr5[5], sb5[5];
+      // the tangents' coordinates and signs of an aligned metric vector
+      constexpr int IL = AXIS == 0 ? 1 : 0, IM = AXIS == 2 ? 1 : 2;
+      constexpr int SL = AXIS == 0 ? 1 : -1, SM = AXIS == 2 ? -1 : 1;
+      const bool sparse = MET == 2 && (row == 1 || row == 2);
+      const int tq = 1 + (row == 1 ? IL : IM);
+      const double sg = row == 1 ? SL : SM;
+      if constexpr (MET == 2) {
+        const double un = a[AXIS], ul = SL > 0 ? a[IL] : -a[IL], um = SM > 0 ? a[IM] : -a[IM];
+        const double V2 = (a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) * 0.5;
+        const double KK = (gamma - 1.0) / (a[3] * a[3]);
+        const double KK1 = KK * 0.5;
+        if (row == 0) {
+          sr5[0] = 1.0 - KK * V2;
+          sr5[4] = -KK;
+#pragma unroll
+          for (int q = 0; q < 3; q++) sr5[1 + q] = KK * a[q];
+        } else if (row < 3) {
+          sr5[0] = row == 1 ? -ul : -um;
+        } else {
+          const double X1 = 1.0 / (2.0 * a[3]);
+          sr5[0] = row == 3 ? KK1 * V2 + X1 * un : KK1 * V2 - X1 * un;
+          sr5[4] = KK1;
+#pragma unroll
+          for (int q = 0; q < 3; q++)
+            sr5[1 + q] = q == AXIS ? (row == 3 ? -X1 : X1) - KK1 * a[q] : -(KK1 * a[q]);
+        }
+        if (row == 0) {
+          sb5[0] = sb5[3] = sb5[4] = 1.0;
+          sb5[1] = sb5[2] = 0.0;
+        } else if (row < 4) {
+          const double v = row == 1 ? a[0] : (row == 2 ? a[1] : a[2]);
+          sb5[0] = v;
+          sb5[1] = row == 1 + IL ? SL : 0.0;
+          sb5[2] = row == 1 + IM ? SM : 0.0;
+          sb5[3] = row == 1 + AXIS ? v - a[3] : v;
+          sb5[4] = row == 1 + AXIS ? v + a[3] : v;
+        } else {
+          const double H = V2 + 1.0 / KK;
+          sb5[0] = V2;
+          sb5[1] = ul;
+          sb5[2] = um;
+          sb5[3] = madd(-a[3], un, H);
+          sb5[4] = madd(a[3], un, H);
+        }
+      } else {
+        CharBasis Bs;
+        char_basis(gamma, a[0], a[1], a[2], a[3], a[4], a[5], a[6], Bs);
+        char_S_row(Bs, row, sr5);
+        char_S1_row(Bs, row, sb5);
+      }
+      // one flux projected (FP64) and reconstructed (RR) at a time, one
+      // component's loads at a time (registers, as in the sweeps).  FP64 path:
+      // the reference's two roundings per term; the mixed form fuses them.
+      auto acc = [](double x, double y, double z) { return sizeof(RR) == 8 ? madd(x, y, z) : fma(x, y, z); };
+      // (points k0 .. k0 + 6: WENO7 of flux + reads 0 .. 6, of flux - 1 .. 7,
+      // WENO5 the inner five; outside its stencil, Ka1_H2.. / Ka1_H3.., the
+      // closures read 0)
+      auto project = [&](int p, const int k0, RR *y) {
+        double x[8];
+#pragma unroll
+        for (int k = k0; k < k0 + 7; k++) x[k] = sr5[0] * double(F[(p * 8 + k) * FB]);
+        if (sparse) {
+#pragma unroll
+          for (int k = k0; k < k0 + 7; k++) x[k] = xmadd(sg, double(F[((p + tq) * 8 + k) * FB]), x[k]);
+        } else {
+#pragma unroll
+          for (int q = 1; q < 5; q++) {
+#pragma unroll
+            for (int k = k0; k < k0 + 7; k++) asm volatile("" : "+v"(x[k]) : : "memory");
+#pragma unroll
+            for (int k = k0; k < k0 + 7; k++) x[k] = acc(sr5[q], double(F[((p + q) * 8 + k) * FB]), x[k]);
+          }
+        }
 #pragma unroll
         for (int k = 0; k < 8; k++) {
-          xp[k] = sF[fb][k * 10 + m];
-          xm[k] = sF[fb][k * 10 + 5 + m];
+          const bool in = k >= k0 && k < k0 + 7;
+          const bool inner = k > k0 && k < k0 + 6;
+          y[k] = in ? RR(x[in ? k : k0]) : RR(0.0);
+          if (!MET && in && !inner && scm == 3) y[k] = RR(0.0);
         }
-        double *o = out + (int64_t)(f0 + fb) * NH;
-        o[m] = double(FAST ? inner_p<SCH_HYBRID>(S, xp, scm) : face_p_nonchar<SCH_HYBRID>(S, xp, s, n, AXIS, scm));
-        o[5 + m] = double(FAST ? inner_m<SCH_HYBRID>(S, xm, scm)
-                               : face_m_nonchar<SCH_HYBRID>(S, xm, s, n, AXIS, scm));
-      }
+      };
+      RR y[8];
+      project(0, 0, y);
+      const RR hp = recon_p(y);
+      __builtin_amdgcn_sched_barrier(0);
+      project(5, 1, y);
+      const RR hm = recon_m(y);
+      sG[row * FB + lane] = double(hp + hm);
+      __syncthreads();
+      // back to conservative components (S1 * h0): component `row`
+      double h0[5];
+#pragma unroll
+      for (int q = 0; q < 5; q++) h0[q] = sG[q * FB + lane];
+      const double hh = madd(sb5[4], h0[4], madd(sb5[3], h0[3], madd(sb5[2], h0[2], madd(sb5[1], h0[1], sb5[0] * h0[0]))));
+      if (f < count) out[(int64_t)f * NH + row] = hh;
     }
-    __syncthreads();  // the next batch overwrites the LDS arrays
   }
 }
 
-// The grid of the striding face kernel: as many workgroups as the device
-// holds at once (CUs x resident workgroups per CU), so that every workgroup
-// runs from the start and the batches spread evenly; a larger grid leaves a
-// tail of workgroups that start late and run nearly alone.  `cache` holds
-// the value per device for one kernel.
+// one axis (AXIS >= 0), or all three in one launch of 3 x nwg workgroups
+template <int AXIS, bool CHAR, int MET, typename RR>
+__global__ __launch_bounds__(WNT) void k_weno_faces(const Block B, const int nwg) {
+  // per batch:
+  __shared__ RR sF[NSUB * 80 * FB];                // [10 components][8 points][face]
+  __shared__ double sQ[CHAR ? NSUB * 14 * FB : 1];  // u, v, w, c, A1..A3 at points s, s+1
+  __shared__ double sG[CHAR ? NSUB * 5 * FB : 1];   // characteristic fluxes h0(1:5)
+  const int wg = (int)blockIdx.x % nwg;
+  const int axis = AXIS >= 0 ? AXIS : (int)blockIdx.x / nwg;
+  if (axis == 0) weno_faces_axis<0, CHAR, MET, RR>(B, sF, sQ, sG, wg, nwg);
+  else if (axis == 1) weno_faces_axis<1, CHAR, MET, RR>(B, sF, sQ, sG, wg, nwg);
+  else weno_faces_axis<2, CHAR, MET, RR>(B, sF, sQ, sG, wg, nwg);
+}
+
+// As many workgroups per axis as the device holds at once (CUs x resident
+// workgroups per CU), so that the batches spread evenly, and no more than the
+// axis can have batches.
 template <typename K>
-dim3 resident_grid(K kernel, int (&cache)[64]) {
+int weno_groups(K kernel, int64_t faces, int (&cache)[64]) {
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
   if (cache[dev] == 0) {
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, NT, 0) != hipSuccess || per < 1) per = 1;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, WNT, 0) != hipSuccess || per < 1) per = 1;
     cache[dev] = cus * per;
   }
-  return dim3((unsigned)cache[dev]);
+  const int64_t most = ((faces + NSUB * FB - 1) / (NSUB * FB) + NXCD - 1) / NXCD * NXCD;
+  return (int)(most < cache[dev] ? most : cache[dev]);
 }
 
-template <int AXIS, bool CHAR, bool FAST, typename RR>
+template <int AXIS, bool CHAR, int MET, typename RR>
 hipError_t weno_launch(const Block &B, hipStream_t st) {
   static int cache[64] = {};
-  hipLaunchKernelGGL((k_weno_faces<AXIS, CHAR, FAST, RR>), resident_grid(k_weno_faces<AXIS, CHAR, FAST, RR>, cache),
-                     dim3(NT), 0, st, B);
+  const Geom &g = B.g;
+  int64_t faces = TileIndex<0>::nfaces(g);
+  if (AXIS != 0 && TileIndex<1>::nfaces(g) > faces) faces = TileIndex<1>::nfaces(g);
+  if (AXIS != 0 && TileIndex<2>::nfaces(g) > faces) faces = TileIndex<2>::nfaces(g);
+  const int nwg = weno_groups(k_weno_faces<AXIS, CHAR, MET, RR>, faces, cache);
+  hipLaunchKernelGGL((k_weno_faces<AXIS, CHAR, MET, RR>), dim3((unsigned)(AXIS >= 0 ? nwg : 3 * nwg)), dim3(WNT), 0,
+                     st, B, nwg);
   return hipGetLastError();
 }
 
-template <int AXIS, typename RR>
-hipError_t weno_axis_as(const Block &B, hipStream_t st) {
-  const bool fast = B.S.iperiodic[AXIS] == 1 && B.M.uniform;
-  if (B.S.is_char)
-    return fast ? weno_launch<AXIS, true, true, RR>(B, st) : weno_launch<AXIS, true, false, RR>(B, st);
-  return fast ? weno_launch<AXIS, false, true, RR>(B, st) : weno_launch<AXIS, false, false, RR>(B, st);
+// FP32 splitting and reconstruction in the mixed-precision form
+template <int AXIS, bool CHAR, int MET>
+hipError_t weno_prec(const Block &B, hipStream_t st) {
+  if (B.prec == OCFD_PREC_MIXED_CODE) return weno_launch<AXIS, CHAR, MET, float>(B, st);
+  return weno_launch<AXIS, CHAR, MET, double>(B, st);
 }
 
-// FP32 splitting and reconstruction in the mixed-precision form
 template <int AXIS>
 hipError_t weno_axis(const Block &B, hipStream_t st) {
-  if (B.prec == OCFD_PREC_MIXED_CODE) return weno_axis_as<AXIS, float>(B, st);
-  return weno_axis_as<AXIS, double>(B, st);
+  if (!(B.S.iperiodic[AXIS] == 1 && B.M.uniform))
+    return B.S.is_char ? weno_prec<AXIS, true, 0>(B, st) : weno_prec<AXIS, false, 0>(B, st);
+  if (!B.S.is_char) return weno_prec<AXIS, false, 1>(B, st);
+  return axis_aligned<AXIS>(B.M) ? weno_prec<AXIS, true, 2>(B, st) : weno_prec<AXIS, true, 1>(B, st);
 }
 
 }  // namespace
@@ -377,10 +419,22 @@ hipError_t launch_hybrid_lists(const Block &B, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_weno_faces(const Block &B, int axis, hipStream_t st) {
-  if (axis == 0) return weno_axis<0>(B, st);
-  if (axis == 1) return weno_axis<1>(B, st);
-  return weno_axis<2>(B, st);
+// the listed faces of the three axes: one launch where the axes run the same
+// kernel (a block of 64^3 has few batches per axis, and the axes' tails
+// overlap), else one per axis
+hipError_t launch_weno_faces(const Block &B, hipStream_t st) {
+  if (!prims_match(B)) return hipErrorInvalidValue;
+  const bool per = B.S.iperiodic[0] == 1 && B.S.iperiodic[1] == 1 && B.S.iperiodic[2] == 1;
+  const bool aligned = axis_aligned<0>(B.M) && axis_aligned<1>(B.M) && axis_aligned<2>(B.M);
+  if (per && B.M.uniform) {
+    if (!B.S.is_char) return weno_prec<-1, false, 1>(B, st);
+    if (aligned) return weno_prec<-1, true, 2>(B, st);
+  } else if (!B.M.uniform || (B.S.iperiodic[0] != 1 && B.S.iperiodic[1] != 1 && B.S.iperiodic[2] != 1)) {
+    return B.S.is_char ? weno_prec<-1, true, 0>(B, st) : weno_prec<-1, false, 0>(B, st);
+  }
+  hipError_t e = weno_axis<0>(B, st);
+  if (e == hipSuccess) e = weno_axis<1>(B, st);
+  return e == hipSuccess ? weno_axis<2>(B, st) : e;
 }
 
 }  // namespace ocfd

@@ -244,6 +244,15 @@ inline int64_t sweep_tiles(const Geom &g, int axis, int shape) {
   return (int64_t)((n + tl - 1) / tl) * ((nw + tw - 1) / tw) * nc;
 }
 
+// whether a uniform grid's metric vector of the axis points along its own
+// coordinate, in the positive direction (every uniform box that is not
+// rotated or skewed)
+template <int AXIS>
+bool axis_aligned(const Metrics &M) {
+  const double *A = &M.u[M_AKX1 + 3 * AXIS];
+  return A[AXIS] > 0.0 && A[(AXIS + 1) % 3] == 0.0 && A[(AXIS + 2) % 3] == 0.0;
+}
+
 // Data of the boundary-layer / swept-corner conditions (ocfd_bc_BoundaryLayer,
 // ocfd_bc_swept_corner, OCFD_BC_Boundarylayers.f90): device arrays the
 // caller provides (ocfd_set_bc_boundarylayer) and the parameters taken from
@@ -314,7 +323,7 @@ int queue_shape(int axis);
 hipError_t launch_batch_queue(const QPlan &P, int prec, int nwg, hipStream_t st);
 // workgroups of the queue kernel resident at once (< 0: query failed)
 int batch_queue_grid(int prec, int device);
-hipError_t launch_weno_faces(const Block &B, int axis, hipStream_t st);
+hipError_t launch_weno_faces(const Block &B, hipStream_t st);
 hipError_t launch_halo_fill(const Block &B, double *const *fields, int nfields, hipStream_t st);
 // the same for primitive fields (at most 5, all of one precision)
 hipError_t launch_halo_prims(const Block &B, const PrimField *fields, int nfields, hipStream_t st);

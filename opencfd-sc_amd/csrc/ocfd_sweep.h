@@ -733,15 +733,6 @@ hipError_t dispatch_march(const Block &B, int mode, int shape, hipStream_t st) {
   }
 }
 
-// whether a uniform grid's metric vector of the axis points along its own
-// coordinate, in the positive direction (every uniform box that is not
-// rotated or skewed)
-template <int AXIS>
-bool axis_aligned(const Metrics &M) {
-  const double *A = &M.u[M_AKX1 + 3 * AXIS];
-  return A[AXIS] > 0.0 && A[(AXIS + 1) % 3] == 0.0 && A[(AXIS + 2) % 3] == 0.0;
-}
-
 template <int AXIS, typename R>
 hipError_t dispatch_axis(const Block &B, int mode, int shape, hipStream_t st) {
   const bool ch = B.S.is_char != 0;
