@@ -41,11 +41,26 @@ constexpr int FNX1 = 2 * FR * FTY, FNX2 = FTX * 2 * FR;    // halo points: 48 be
 constexpr int FQ = 2 * FR + 1;
 constexpr int FKSEG_MAX = 64;
 
-// workgroups and planes per workgroup of the fused march over block g
-inline int fused_kseg(const Geom &g) {
+// Planes per workgroup of the fused march: as march_kseg, the length with the
+// smallest product of rounds of resident workgroups and planes per workgroup
+// -- a segment also runs 2 x 3 planes of Ev3 around it and a prologue of about
+// 2.  A target of 2048 workgroups, at least 16 planes each, left 64^3 on 32
+// CUs (76 us against 32 now) and 96^3 on 72 in six rounds' time (81 / 63); at
+// 192^3 it ran 22 planes per 16 (380 / 352), at 256^3 the choices tie.
+inline int fused_kseg(const Geom &g, int slots) {
   const int64_t cols = (int64_t)(g.nx / FTX) * (g.ny / FTY);
-  const int64_t k = cols * g.nz / 2048;
-  return (int)(k < 16 ? (g.nz < 16 ? g.nz : 16) : (k > FKSEG_MAX ? FKSEG_MAX : k));
+  const int kmax = g.nz < FKSEG_MAX ? g.nz : FKSEG_MAX;
+  int best = kmax;
+  int64_t cost = INT64_MAX;
+  for (int k = kmax; k >= 1; k--) {
+    const int64_t groups = cols * ((g.nz + k - 1) / k);
+    const int64_t c = (groups + slots - 1) / slots * (k + 2 * FR + 2);
+    if (c < cost) {
+      cost = c;
+      best = k;
+    }
+  }
+  return best;
 }
 inline unsigned fused_blocks(const Geom &g, int kseg) {
   return (unsigned)((g.nx / FTX) * (g.ny / FTY) * ((g.nz + kseg - 1) / kseg));
@@ -360,7 +375,8 @@ hipError_t visc_fused_as(const Block &B, int krk, int refresh, int *neg, hipStre
   if (g.nx % FTX != 0 || g.ny % FTY != 0 || !all_periodic(B) || B.S.scheme_vis == SCH_CD8 || !B.u2.p ||
       !B.v2.p || !B.w2.p)
     return hipErrorInvalidValue;
-  const int kseg = fused_kseg(g);
+  static int cache[64] = {};
+  const int kseg = fused_kseg(g, resident_groups(k_visc_fused<RT>, cache));
   hipLaunchKernelGGL(k_visc_fused<RT>, dim3(fused_blocks(g, kseg)), dim3(NT), 0, st, B, krk, refresh, kseg, neg);
   return hipGetLastError();
 }
