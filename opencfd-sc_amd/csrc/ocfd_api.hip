@@ -69,6 +69,10 @@ struct ocfd_handle {
   int tpar = 0;
   int uvpar = 0;
   bool fused = false;              // stages run k_visc_fused (Block::u2, v2, w2 allocated)
+  // periodic on every axis, no boundary or ghost kernel: the halo fill of a
+  // stage is all that writes halos, so it writes both buffers of T (u, v, w)
+  // and the repair copies none (mixed 256^3: repair 61 -> 4 us per stage)
+  bool halo_both = false;
   // per-routine calls merged into the whole-step stage kernels
   // (ocfd_set_stage_fusion); pend holds what the stage so far left to do
   bool stage_fusion = false;
@@ -325,6 +329,22 @@ int prim_upload(ocfd_handle *h, int q, const double *src) {
   return 0;
 }
 
+// the second buffers of T and u, v, w hold the halos (edges and corners
+// included) of the first after an upload (ocfd_handle::halo_both)
+int copy_second(ocfd_handle *h) {
+  if (!h->halo_both) return 0;
+  const Block &B = h->B;
+  const size_t n = (size_t)B.g.nh * (B.T.f32 ? sizeof(float) : sizeof(double));
+  HIPCHK(hipMemcpyAsync(B.T2.p, B.T.p, n, hipMemcpyDeviceToDevice, h->st));
+  if (h->fused) {
+    HIPCHK(hipMemcpyAsync(B.u2.p, B.u.p, n, hipMemcpyDeviceToDevice, h->st));
+    HIPCHK(hipMemcpyAsync(B.v2.p, B.v.p, n, hipMemcpyDeviceToDevice, h->st));
+    HIPCHK(hipMemcpyAsync(B.w2.p, B.w.p, n, hipMemcpyDeviceToDevice, h->st));
+  }
+  HIPCHK(hipStreamSynchronize(h->st));
+  return 0;
+}
+
 // the primitives from nh doubles per field on the host; with make_f, f from
 // those FP64 values as at start-up (init3d, OCFD_init.f90:10-20).  In the
 // mixed-precision form the FP64 values pass through device scratch fields, so
@@ -336,6 +356,7 @@ int upload_prims(ocfd_handle *h, const double *const src[5], bool make_f) {
     for (int q = 0; q < 5; q++)
       if (prim_upload(h, q, src[q])) return -1;
     if (make_f && launch(h, "init_f", [&] { return launch_init_f(h->B, h->st); })) return -1;
+    if (copy_second(h)) return -1;
     HIPCHK(hipStreamSynchronize(h->st));
     return 0;
   }
@@ -355,6 +376,7 @@ int upload_prims(ocfd_handle *h, const double *const src[5], bool make_f) {
       if (f64[q]->p) (void)hipFree(f64[q]->p);
   }
   for (int q = 0; q < 5 && !rc; q++) rc = prim_upload(h, q, src[q]);
+  if (!rc) rc = copy_second(h);
   return rc;
 }
 
@@ -374,6 +396,11 @@ int inviscid(ocfd_handle *h, bool ch) {
     if (launch(h, nm[ch][a], [&] { return launch_inviscid(B, a, modes[a], SweepTile{h->tile[a]}, h->st); }))
       return -1;
   return 0;
+}
+
+// the halo fill at the start of a whole step's stage
+int exchange_stage(ocfd_handle *h) {
+  return launch(h, "halo_fill", [&] { return launch_halo_both(h->B, h->st); });
 }
 
 int exchange_prims(ocfd_handle *h) {
@@ -453,7 +480,7 @@ void swap_uvw(ocfd_handle *h) {
 }
 
 // ocfd_handle::pend bits (stage fusion)
-constexpr int PEND_VISC = 1, PEND_UPDATE = 2, PEND_REFRESHED = 4, PEND_UVW = 8;
+constexpr int PEND_VISC = 1, PEND_UPDATE = 2, PEND_REFRESHED = 4, PEND_UVW = 8, PEND_HALO = 16;
 
 int read_neg(ocfd_handle *h, int out[3]) {
   HIPCHK(hipMemcpyAsync(out, h->neg, sizeof(int), hipMemcpyDeviceToHost, h->st));
@@ -500,6 +527,8 @@ int ocfd_create(const ocfd_config *cfg, int device, ocfd_handle **out) {
   h->fused = cfg->if_viscous == 1 && cfg->ibc == 0 && visc_fused_supported(B) &&
              std::getenv("OCFD_NO_FUSED") == nullptr;
   for (int q = 0; q < 6; q++) h->fused = h->fused && cfg->ghost_cell[q] == 0;
+  h->halo_both = cfg->ibc == 0 && cfg->iperiodic[0] == 1 && cfg->iperiodic[1] == 1 && cfg->iperiodic[2] == 1;
+  for (int q = 0; q < 6; q++) h->halo_both = h->halo_both && cfg->ghost_cell[q] == 0;
   if (h->fused)
     for (PrimField *p : {&B.u2, &B.v2, &B.w2}) rc |= alloc_prim(p, B.g.nh, p32);
   B.halt = nullptr;
@@ -844,7 +873,13 @@ int ocfd_get_time(ocfd_handle *h, int32_t *istep, double *tt) {
 }
 
 // ---- one reference routine each ---------------------------------------------
-int ocfd_exchange_primitives(ocfd_handle *h) { return exchange_prims(h); }
+int ocfd_exchange_primitives(ocfd_handle *h) {
+  if (h->stage_fusion && h->halo_both) {
+    h->pend |= PEND_HALO;
+    return exchange_stage(h);
+  }
+  return exchange_prims(h);
+}
 
 int ocfd_comput_rhybrid(ocfd_handle *h, int64_t counts[4]) {
   if (!h->B.rhyb) return fail("comput_Rhybrid needs the HYBRID scheme");
@@ -886,7 +921,7 @@ int ocfd_time_adv_rk3(ocfd_handle *h, int32_t krk) {
     hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(128), 0, h->st, h->neg, NEG_STRIDE);
     const int refresh = h->ibc == 0 ? 1 : 0;
     const bool visc = (h->pend & PEND_VISC) != 0;
-    int pend = PEND_UPDATE | (refresh ? PEND_REFRESHED : 0);
+    int pend = PEND_UPDATE | (refresh ? PEND_REFRESHED : 0) | (h->pend & PEND_HALO);
     if (visc && h->fused) {
       if (launch(h, "stage_update_fused", [&] { return launch_visc_fused(h->B, krk, refresh, h->neg, h->st); }))
         return -1;
@@ -919,9 +954,10 @@ int ocfd_comput_duvwt(ocfd_handle *h) {
   if (h->stage_fusion && (h->pend & PEND_UPDATE)) {
     // primitives already recovered by the stage update: repair and count
     const int uvw = (h->pend & PEND_UVW) ? 1 : 0;
-    if (launch(h, "negt_repair", [&] { return launch_negt_repair(h->B, h->neg, h->st, uvw); })) return -1;
+    const bool copy = (h->pend & PEND_HALO) == 0;
+    if (launch(h, "negt_repair", [&] { return launch_negt_repair(h->B, h->neg, h->st, uvw, copy); })) return -1;
     swap_T(h);
-    h->pend &= ~(PEND_UPDATE | PEND_UVW);
+    h->pend &= ~(PEND_UPDATE | PEND_UVW | PEND_HALO);
     int c[3];
     if (read_neg(h, c)) return -1;
     return c[1];
@@ -1057,7 +1093,7 @@ int step_body(ocfd_handle *h) {
   const bool hyb = c.scheme_invis == SCH_HYBRID;
   const bool ch = c.if_scheme_character != 0;
   for (int krk = 1; krk <= 3; krk++) {
-    if (exchange_prims(h)) return -1;
+    if (h->halo_both ? exchange_stage(h) : exchange_prims(h)) return -1;
     if (krk == 1 && hyb && sensor(h)) return -1;
     if (inviscid(h, ch)) return -1;
     const int refresh = h->ibc == 0 ? 1 : 0;
@@ -1074,7 +1110,7 @@ int step_body(ocfd_handle *h) {
         return -1;
     }
     const int uvw = h->fused ? 1 : 0;
-    if (launch(h, "negt_repair", [&] { return launch_negt_repair(h->B, h->neg, h->st, uvw); })) return -1;
+    if (launch(h, "negt_repair", [&] { return launch_negt_repair(h->B, h->neg, h->st, uvw, !h->halo_both); })) return -1;
     swap_T(h);
     if (h->ibc != 0) {
       if ((h->ibc == 2 || h->ibc == 3) && !h->bl_set)
@@ -1379,7 +1415,6 @@ struct ocfd_batch {
   std::vector<SweepGroup> sweep;
   std::vector<ViscGroup> vis;
   Launch halo;
-  Launch hcopy;               // the T -> T2 halo copies after each stage update
   bool use_graph = true;
   hipGraphExec_t gexec[2] = {nullptr, nullptr};  // one step starting from table [q]
   int64_t cells = 0;
@@ -1400,8 +1435,8 @@ struct ocfd_batch {
 
 namespace {
 
-BoxSet boxset(const ocfd_batch *b, const ocfd_batch::Launch &l, int table = 0, bool repair = false) {
-  return BoxSet{repair ? b->drep[table] : b->dblk[table], b->dtab + l.ids, b->dtab + l.off, l.m};
+BoxSet boxset(const ocfd_batch *b, const ocfd_batch::Launch &l, int table = 0) {
+  return BoxSet{b->dblk[table], b->dtab + l.ids, b->dtab + l.off, l.m};
 }
 
 // box list + tile offsets of one launch, appended to the host table
@@ -1486,8 +1521,7 @@ int batch_step_body(ocfd_batch *b, int q0) {
                                                  (int)l.ntiles, b->st);
       if (e != hipSuccess) return fail(std::string("batched stage update: ") + hipGetErrorString(e));
     }
-    const hipError_t e = launch_negt_repair_batch(boxset(b, b->hcopy, q, true), (int)b->box.size(), b->neg,
-                                                  (int)b->hcopy.ntiles, b->st);
+    const hipError_t e = launch_negt_repair_batch(b->drep[q], (int)b->box.size(), b->neg, b->st);
     if (e != hipSuccess) return fail(std::string("batched T <= 0 repair: ") + hipGetErrorString(e));
   }
   return 0;
@@ -1713,7 +1747,6 @@ int ocfd_batch_create(const ocfd_config *cfgs, int32_t nbox, int32_t device, ocf
   std::vector<int> all(nbox);
   for (int i = 0; i < nbox; i++) all[i] = i;
   b->halo = add_launch(b, all, [](const Geom &g) { return halo_tiles(g); });
-  b->hcopy = add_launch(b, all, [](const Geom &g) { return halo_copy_tiles(g); });
   b->qrep = add_launch(b, all, [](const Geom &g) { return 1 + halo_copy_tiles(g); });
   // the queue kernel runs the non-characteristic sweeps and CD6
   b->queue_ok = true;

@@ -280,11 +280,8 @@ hipError_t launch_visc_flux_batch(const BoxSet &S, int prec, bool cd8, int ntile
 hipError_t launch_visc_div_update_batch(const BoxSet &S, int prec, bool visc, bool cd8, int krk, int *neg,
                                         int ntiles, hipStream_t st);
 hipError_t launch_halo_batch(const BoxSet &S, int ntiles, hipStream_t st);
-// the T <= 0 repair of every box (workgroup b repairs box b of the table) and
-// the copy of T's halo into T2, over the halo-copy tiles of S (for boxes
-// with second u, v, w buffers, i.e. a fused stage, also the halos of u2, v2,
-// w2 into u, v, w)
-hipError_t launch_negt_repair_batch(const BoxSet &S, int nbox, int *neg, int ntiles, hipStream_t st);
+// the T <= 0 repair of every box of the table blk
+hipError_t launch_negt_repair_batch(const Block *blk, int nbox, int *neg, hipStream_t st);
 // workgroups of the T -> T2 halo copy of one box
 int64_t halo_copy_tiles(const Geom &g);
 // workgroups of the k-marching kernels of a block marched in segments of
@@ -327,6 +324,9 @@ hipError_t launch_weno_faces(const Block &B, hipStream_t st);
 hipError_t launch_halo_fill(const Block &B, double *const *fields, int nfields, hipStream_t st);
 // the same for primitive fields (at most 5, all of one precision)
 hipError_t launch_halo_prims(const Block &B, const PrimField *fields, int nfields, hipStream_t st);
+// the five primitives, T also into T2 and u, v, w into u2, v2, w2 where they
+// exist: the repair after the stage then has no halos to copy
+hipError_t launch_halo_both(const Block &B, hipStream_t st);
 hipError_t launch_sensor(const Block &B, hipStream_t st);
 hipError_t launch_sensor2(const Block &B, double *work, hipStream_t st);
 hipError_t launch_hybrid_counts(const Block &B, unsigned long long *counts, hipStream_t st);
@@ -340,7 +340,8 @@ hipError_t launch_duvwt(const Block &B, int *neg, hipStream_t st);
 // the copy of T's halo into T2, in one launch
 // (uvw: also copy the halos of u2, v2, w2 into u, v, w -- after a fused
 // stage, whose new u, v, w the host has swapped in)
-hipError_t launch_negt_repair(const Block &B, int *neg, hipStream_t st, int uvw = 0);
+// (copy = false: launch_halo_both has filled both buffers' halos)
+hipError_t launch_negt_repair(const Block &B, int *neg, hipStream_t st, int uvw = 0, bool copy = true);
 // the viscous terms fused into the stage update (k_visc_fused): whether this
 // block can take it, and the launch (writes u2, v2, w2 and T2)
 bool visc_fused_supported(const Block &B);

@@ -18,18 +18,20 @@ inline unsigned nb(int64_t n) { return (unsigned)((n + NT - 1) / NT); }
 
 __global__ void k_halo(const Geom g, const HaloFields F, const int nf, const int px, const int py, const int pz) {
   const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-  if (F.f32) halo_point<float>(g, F.p, nf, px, py, pz, t);
-  else halo_point<double>(g, F.p, nf, px, py, pz, t);
+  if (F.f32) halo_point<float>(g, F.p, nf, px, py, pz, t, F.p2);
+  else halo_point<double>(g, F.p, nf, px, py, pz, t, F.p2);
 }
 
-// the five primitives of every box of a batch (all axes periodic)
+// the five primitives of every box of a batch (all axes periodic), those with
+// a second buffer into both
 __global__ __launch_bounds__(NT) void k_halo_batch(const BoxSet S) {
   const int j = S.entry(blockIdx.x);
   const Block &B = S.blk[S.ids[j]];
   void *const P[5] = {B.d.p, B.u.p, B.v.p, B.w.p, B.T.p};
   const int64_t t = (int64_t)(blockIdx.x - S.off[j]) * NT + threadIdx.x;
-  if (B.d.f32) halo_point<float>(B.g, P, 5, 1, 1, 1, t);
-  else halo_point<double>(B.g, P, 5, 1, 1, 1, t);
+  void *const P2[5] = {nullptr, B.u2.p, B.v2.p, B.w2.p, B.T2.p};
+  if (B.d.f32) halo_point<float>(B.g, P, 5, 1, 1, 1, t, P2);
+  else halo_point<double>(B.g, P, 5, 1, 1, 1, t, P2);
 }
 
 // ---------------------------------------------------------------------------
@@ -258,17 +260,10 @@ __global__ __launch_bounds__(NT) void k_negt_repair(const Block B, int *neg, con
   halo_copy_tile(B, blockIdx.x - 1, uvw);
 }
 
-// batches: workgroup b < nbox repairs box b (its counters at neg + NEG_STRIDE
-// * b); the others copy halos over the tiles of S
-__global__ __launch_bounds__(NT) void k_negt_repair_batch(const BoxSet S, const int nbox, int *neg) {
-  if ((int)blockIdx.x < nbox) {
-    if (threadIdx.x == 0) negt_repair_body(S.blk[blockIdx.x], neg + NEG_STRIDE * blockIdx.x, 1);
-    return;
-  }
-  const int t = blockIdx.x - nbox;
-  const int j = S.entry(t);
-  const Block &B = S.blk[S.ids[j]];
-  halo_copy_tile(B, t - S.off[j], B.u2.p != nullptr ? 1 : 0);
+// batches: workgroup b repairs box b (its counters at neg + NEG_STRIDE * b);
+// the halo fill has written both buffers
+__global__ __launch_bounds__(64) void k_negt_repair_batch(const Block *blk, int *neg) {
+  if (threadIdx.x == 0) negt_repair_body(blk[blockIdx.x], neg + NEG_STRIDE * blockIdx.x, 1);
 }
 
 // ---------------------------------------------------------------------------
@@ -846,7 +841,8 @@ __global__ __launch_bounds__(NT) void k_normalise(const Geom g, const MetPtrs mp
 // launchers
 // ---------------------------------------------------------------------------
 namespace {
-hipError_t halo_fill(const Block &B, void *const *fields, int nfields, int f32, hipStream_t st) {
+hipError_t halo_fill(const Block &B, void *const *fields, int nfields, int f32, hipStream_t st,
+                     void *const *second = nullptr) {
   const Geom &g = B.g;
   const int px = B.S.iperiodic[0] == 1, py = B.S.iperiodic[1] == 1, pz = B.S.iperiodic[2] == 1;
   const int64_t tot = (px ? (int64_t)2 * LAP * g.ny * g.nz : 0) + (py ? (int64_t)2 * LAP * g.nx * g.nz : 0) +
@@ -855,7 +851,10 @@ hipError_t halo_fill(const Block &B, void *const *fields, int nfields, int f32, 
   for (int f0 = 0; f0 < nfields; f0 += 8) {
     HaloFields F;
     const int nf = nfields - f0 < 8 ? nfields - f0 : 8;
-    for (int q = 0; q < nf; q++) F.p[q] = fields[f0 + q];
+    for (int q = 0; q < nf; q++) {
+      F.p[q] = fields[f0 + q];
+      F.p2[q] = second ? second[f0 + q] : nullptr;
+    }
     F.f32 = f32;
     hipLaunchKernelGGL(k_halo, dim3(nb(tot)), dim3(NT), 0, st, g, F, nf, px, py, pz);
   }
@@ -878,6 +877,13 @@ hipError_t launch_halo_prims(const Block &B, const PrimField *fields, int nfield
     p[q] = fields[q].p;
   }
   return halo_fill(B, p, nfields, fields[0].f32, st);
+}
+
+hipError_t launch_halo_both(const Block &B, hipStream_t st) {
+  if (!prims_match(B)) return hipErrorInvalidValue;
+  void *const p[5] = {B.d.p, B.u.p, B.v.p, B.w.p, B.T.p};
+  void *const p2[5] = {nullptr, B.u2.p, B.v2.p, B.w2.p, B.T2.p};
+  return halo_fill(B, p, 5, B.d.f32, st, p2);
 }
 
 hipError_t launch_sensor(const Block &B, hipStream_t st) {
@@ -936,8 +942,8 @@ hipError_t launch_halo_batch(const BoxSet &S, int ntiles, hipStream_t st) {
 
 int64_t halo_copy_tiles(const Geom &g) { return halo_copy_tiles_of(g); }
 
-hipError_t launch_negt_repair_batch(const BoxSet &S, int nbox, int *neg, int ntiles, hipStream_t st) {
-  hipLaunchKernelGGL(k_negt_repair_batch, dim3((unsigned)(nbox + ntiles)), dim3(NT), 0, st, S, nbox, neg);
+hipError_t launch_negt_repair_batch(const Block *blk, int nbox, int *neg, hipStream_t st) {
+  hipLaunchKernelGGL(k_negt_repair_batch, dim3((unsigned)nbox), dim3(64), 0, st, blk, neg);
   return hipGetLastError();
 }
 
@@ -947,9 +953,10 @@ hipError_t launch_cfl_rate(const Block &B, unsigned long long *out, hipStream_t 
   return hipGetLastError();
 }
 
-hipError_t launch_negt_repair(const Block &B, int *neg, hipStream_t st, int uvw) {
+hipError_t launch_negt_repair(const Block &B, int *neg, hipStream_t st, int uvw, bool copy) {
   if (uvw && (!B.u2.p || !B.v2.p || !B.w2.p)) return hipErrorInvalidValue;
-  hipLaunchKernelGGL(k_negt_repair, dim3((unsigned)(1 + halo_copy_tiles_of(B.g))), dim3(NT), 0, st, B, neg, 1, uvw);
+  hipLaunchKernelGGL(k_negt_repair, dim3((unsigned)(1 + (copy ? halo_copy_tiles_of(B.g) : 0))), dim3(NT), 0, st, B, neg,
+                     1, uvw);
   return hipGetLastError();
 }
 

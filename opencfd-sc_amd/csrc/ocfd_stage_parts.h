@@ -15,11 +15,12 @@ namespace {
 // ---------------------------------------------------------------------------
 struct HaloFields {
   void *p[8];
+  void *p2[8];  // second destination of each field, or NULL
   int f32;  // float fields (primitives of the mixed-precision form)
 };
 template <typename E>
 __device__ inline void halo_point(const Geom &g, void *const *P, const int nf, const int px, const int py,
-                                  const int pz, const int64_t t) {
+                                  const int pz, const int64_t t, void *const *P2 = nullptr) {
   const int64_t nxh = px ? (int64_t)2 * LAP * g.ny * g.nz : 0;
   const int64_t nyh = py ? (int64_t)2 * LAP * g.nx * g.nz : 0;
   const int64_t nzh = pz ? (int64_t)2 * LAP * g.nx * g.ny : 0;
@@ -47,7 +48,11 @@ __device__ inline void halo_point(const Geom &g, void *const *P, const int nf, c
     if (l < LAP) { dst = g.hi(i, j, g.nz + 1 + l); src = g.hi(i, j, 1 + l); }
     else { const int q = l - LAP; dst = g.hi(i, j, 1 - LAP + q); src = g.hi(i, j, g.nz - LAP + 1 + q); }
   }
-  for (int q = 0; q < nf; q++) static_cast<E *>(P[q])[dst] = static_cast<E *>(P[q])[src];
+  for (int q = 0; q < nf; q++) {
+    const E v = static_cast<E *>(P[q])[src];
+    static_cast<E *>(P[q])[dst] = v;
+    if (P2 && P2[q]) static_cast<E *>(P2[q])[dst] = v;
+  }
 }
 
 // T <= 0 repair (handle_NegativeT, OCFD_handle_NegativeT.f90:11, called from
@@ -103,7 +108,9 @@ __device__ void negt_repair_body(const Block &B, int *neg, const int refresh) {
 }
 
 // Copy of T's halo points into T2 (the stage update and comput_duvwT write
-// the interior of T2 only).  Tile q of a box covers HCOPY_ROWS (j, k) rows
+// the interior of T2 only).  Whole steps of periodic blocks do without it:
+// there the stage's halo fill writes both buffers, which are alike at the
+// edges and corners it does not touch (an upload fills both).  Tile q of a box covers HCOPY_ROWS (j, k) rows
 // of the halo'd array: rows outside the interior j, k range are copied whole,
 // the others at their 2 * LAP i-halo points.
 constexpr int HCOPY_ROWS = 16;
