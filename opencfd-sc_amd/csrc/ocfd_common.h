@@ -138,6 +138,10 @@ __device__ inline double wdiv(double a, double b) {
   return __builtin_amdgcn_div_fixup(__builtin_fma(__builtin_fma(-b, q, a), y, q), b, a);
 }
 __device__ inline float wdiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+// IEEE a / b for operands far from the ends of the range: FP64 as wdiv, so
+// quotients of one divisor share its reciprocal; FP32 the division itself
+__device__ inline double ediv(double a, double b) { return wdiv(a, b); }
+__device__ inline float ediv(float a, float b) { return a / b; }
 // a / b for a divisor known in advance, rb = 1 / b correctly rounded: the
 // quotient and one remainder correction give the correctly rounded a / b
 // (Markstein; Brisebarre, Muller and Raina, "Accelerating correctly rounded
@@ -634,14 +638,15 @@ typedef CharBasisT<double> CharBasis;
 template <typename T>
 __device__ inline void char_basis(T gamma, T u1, T v1, T w1, T c1, T a1, T a2,
                                   T a3, CharBasisT<T> &B) {
+  // (8 quotients, 3 + 2 of them with one divisor)
   T ss = sqrt(a1 * a1 + a2 * a2 + a3 * a3);
-  B.n1 = a1 / ss; B.n2 = a2 / ss; B.n3 = a3 / ss;
+  B.n1 = ediv(a1, ss); B.n2 = ediv(a2, ss); B.n3 = ediv(a3, ss);
   if (fabs(B.n3) <= fabs(B.n2)) {
     ss = sqrt(B.n1 * B.n1 + B.n2 * B.n2);
-    B.l1 = -B.n2 / ss; B.l2 = B.n1 / ss; B.l3 = T(0.0);
+    B.l1 = ediv(-B.n2, ss); B.l2 = ediv(B.n1, ss); B.l3 = T(0.0);
   } else {
     ss = sqrt(B.n1 * B.n1 + B.n3 * B.n3);
-    B.l1 = -B.n3 / ss; B.l2 = T(0.0); B.l3 = B.n1 / ss;
+    B.l1 = ediv(-B.n3, ss); B.l2 = T(0.0); B.l3 = ediv(B.n1, ss);
   }
   B.m1 = B.n2 * B.l3 - B.n3 * B.l2;
   B.m2 = B.n3 * B.l1 - B.n1 * B.l3;
@@ -650,10 +655,10 @@ __device__ inline void char_basis(T gamma, T u1, T v1, T w1, T c1, T a1, T a2,
   B.ul = u1 * B.l1 + v1 * B.l2 + w1 * B.l3;
   B.um = u1 * B.m1 + v1 * B.m2 + w1 * B.m3;
   B.V2 = (u1 * u1 + v1 * v1 + w1 * w1) * T(0.5);
-  B.KK = (gamma - T(1.0)) / (c1 * c1);
+  B.KK = ediv(gamma - T(1.0), c1 * c1);
   B.KK1 = B.KK * T(0.5);
-  B.X1 = T(1.0) / (T(2.0) * c1);
-  B.H = B.V2 + T(1.0) / B.KK;
+  B.X1 = ediv(T(1.0), T(2.0) * c1);
+  B.H = B.V2 + ediv(T(1.0), B.KK);
   B.u1 = u1; B.v1 = v1; B.w1 = w1; B.c1 = c1;
 }
 // row r of S (OCFD_inviscous_character.f90:238-242)

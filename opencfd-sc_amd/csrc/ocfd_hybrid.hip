@@ -17,6 +17,8 @@
 // same expression as in the sweep (flux_charteric,
 // OCFD_inviscous_character.f90:190-290; OCFD2d_flux1/2,
 // OCFD_inviscous.f90:210-361), so results are unchanged bit for bit.
+#include <type_traits>
+
 #include "ocfd_kernels.h"
 
 namespace ocfd {
@@ -32,37 +34,46 @@ constexpr int WNT = NSUB * 5 * FB;  // per batch a wavefront for each characteri
 // face -> slot map.  The list position is reserved with one atomic per
 // workgroup; inside it the slots follow the face index.
 constexpr int LPT = 16;  // faces per thread
+constexpr int LPB = 8;   // of which the sensor values are loaded together
 template <int AXIS>
-__global__ __launch_bounds__(NT) void k_hyb_list(const Block B) {
+__device__ __forceinline__ void hyb_list_axis(const Block &B, int (&soff)[LPT][NT / 64], int &sbase, const int64_t blk) {
   typedef TileIndex<AXIS> TI;
-  __shared__ int soff[LPT][NT / 64];
-  __shared__ int sbase;
   const Geom &g = B.g;
   const SchemeParams &S = B.S;
   const int n = g.n(AXIS);
   const int64_t nfa = TI::nfaces(g);
-  const int64_t f0 = (int64_t)blockIdx.x * (NT * LPT) + threadIdx.x;
+  const int64_t f0 = blk * (NT * LPT) + threadIdx.x;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   unsigned wbits = 0, hbits = 0;  // bit it: face f0 + it * NT is WENO / WENO7-class
-  for (int it = 0; it < LPT; it++) {
-    const int64_t fid = f0 + (int64_t)it * NT;
-    bool weno = false;
-    if (fid < nfa) {
-      int s, w, c;
-      TI::face_of(g, fid, s, w, c);
+#pragma unroll 1
+  for (int i0 = 0; i0 < LPT; i0 += LPB) {
+    // the sensor values of LPB faces before the first is looked at
+    double ra[LPB], rb[LPB];
+    int sv[LPB];
+#pragma unroll
+    for (int q = 0; q < LPB; q++) {
+      const int64_t fid = f0 + (int64_t)(i0 + q) * NT;
+      int w, c;
+      TI::face_of(g, fid < nfa ? fid : nfa - 1, sv[q], w, c);
+      const int64_t h = TI::hidx(g, sv[q], w, c);
+      ra[q] = B.rhyb[h];
+      rb[q] = B.rhyb[h + g.hstride(AXIS)];
+    }
+#pragma unroll
+    for (int q = 0; q < LPB; q++) {
+      const int it = i0 + q, s = sv[q];
       // set_hybrid_scheme: the larger sensor value of the two cells of the face
-      const double r0 = dmax2(B.rhyb[TI::hidx(g, s, w, c)], B.rhyb[TI::hidx(g, s + 1, w, c)]);
-      const int scm = hybrid_index(r0, S.hyb2, S.hyb3);
+      const int scm = hybrid_index(dmax2(ra[q], rb[q]), S.hyb2, S.hyb3);
       // the characteristic path closes non-periodic block edges with the
       // non-reflecting face whatever the scheme index
       const bool closure = S.is_char && ((S.bidx[AXIS][0] == 1 && S.sb[2 * AXIS] == 0 && s == 0) ||
                                          (S.bidx[AXIS][1] == 1 && S.sb[2 * AXIS + 1] == 0 && s == n));
-      weno = scm >= 2 && !closure;
+      const bool weno = f0 + (int64_t)it * NT < nfa && scm >= 2 && !closure;
       if (weno) wbits |= 1u << it;
       if (scm == 3) hbits |= 1u << it;
+      const unsigned long long mask = __ballot(weno);
+      if (lane == 0) soff[it][wave] = __popcll(mask);
     }
-    const unsigned long long mask = __ballot(weno);
-    if (lane == 0) soff[it][wave] = __popcll(mask);
   }
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -92,6 +103,22 @@ __global__ __launch_bounds__(NT) void k_hyb_list(const Block B) {
   }
 }
 
+// the lists of the three axes: workgroups [0, n0) x, [n0, n0 + n1) y, then z
+// (256^3 184 us in three launches with one face's loads at a time, 155 now;
+// 101 x 75 x 54 35 and 11.5)
+__global__ __launch_bounds__(NT) void k_hyb_list(const Block B, const unsigned n0, const unsigned n1) {
+  __shared__ int soff[LPT][NT / 64];
+  __shared__ int sbase;
+  if (blockIdx.x < n0) hyb_list_axis<0>(B, soff, sbase, blockIdx.x);
+  else if (blockIdx.x < n0 + n1) hyb_list_axis<1>(B, soff, sbase, blockIdx.x - n0);
+  else hyb_list_axis<2>(B, soff, sbase, blockIdx.x - n0 - n1);
+}
+
+// type the split fluxes are held in: the projections are FP64 in both forms, so
+// the mixed form's FP32 fluxes are widened once instead of by all five rows
+template <bool CHAR, typename RR>
+using weno_lds_t = typename std::conditional<CHAR, double, RR>::type;
+
 // Fluxes of the listed faces of one axis: workgroup wg of nwg strides over
 // batches of FB faces; the list length is read from the device counter.  RR is
 // the real type of the splitting and the WENO reconstruction: double, or float
@@ -115,10 +142,11 @@ __global__ __launch_bounds__(NT) void k_hyb_list(const Block B) {
 // Bound by instruction issue (VALU 65% busy).  256^3, 5.7% of the faces, three
 // axes: FP64 780 us in the former layout (256 lanes on 51 faces, one lane per
 // row: every lane formed all rows' entries, three launches), 695 with five
-// wavefronts per workgroup, 557 now; mixed (8.3%) 705, 550, 541; 160^3 FP64
-// with metric fields (8.6%) 414, 372, 323.
+// wavefronts per workgroup, 527 now; mixed (8.3%) 705, 550, 516; 160^3 FP64
+// with metric fields (8.6%) 414, 372, 305.
 template <int AXIS, bool CHAR, int MET, typename RR>
-__device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, double *const sQa, double *const sGa,
+__device__ __forceinline__ void weno_faces_axis(const Block &B, weno_lds_t<CHAR, RR> *const sFa, double *const sQa,
+                                                double *const sGa,
                                                 const int wg, const int nwg) {
   typedef TileIndex<AXIS> TI;
   constexpr int NH = CHAR ? 5 : 10;
@@ -128,7 +156,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int sub = wave / 5, row = wave - 5 * sub;
-  RR *const sF = sFa + sub * (80 * FB);
+  weno_lds_t<CHAR, RR> *const sF = sFa + sub * (80 * FB);
   double *const sQ = sQa + sub * (CHAR ? 14 * FB : 0), *const sG = sGa + sub * (CHAR ? 5 * FB : 0);
   const int q1 = M_AKX1 + 3 * AXIS;
   const int count = B.hcount[AXIS];
@@ -154,10 +182,13 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
   };
   // stencil points row and row + 5 (< 8) of this lane's face
   RR pv[2][5];
+  int sn = 0;        // the fetched face's s, and its first stencil point
+  int64_t hn = 0;
+  const int64_t st = g.hstride(AXIS);
   auto fetch = [&](int code) {
-    int s, w, c;
-    TI::face_of(g, code >> 1, s, w, c);
-    const int64_t h0 = TI::hidx(g, s - 3, w, c), st = g.hstride(AXIS);
+    int w, c;
+    TI::face_of(g, code >> 1, sn, w, c);
+    const int64_t h0 = hn = TI::hidx(g, sn - 3, w, c);
 #pragma unroll
     for (int r = 0; r < 2; r++)
       if (row + 5 * r < 8) {
@@ -170,8 +201,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
   fetch(code);
   int code1 = entry(b0 + bstep < bhi ? b0 + bstep : b0);
   for (int batch = b0; batch < bhi; batch += bstep) {
-    int s, w, c;
-    TI::face_of(g, code >> 1, s, w, c);
+    const int s = sn;
     // split fluxes at the stencil points (OCFD_inviscous.f90:64-70, split_*)
 #pragma unroll
     for (int r = 0; r < 2; r++) {
@@ -181,7 +211,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
       SplitK<RR> K = split_const<RR>(B, AXIS);
       double A[3] = {0.0, 0.0, 0.0};
       if (!unif) {
-        const int64_t h = TI::hidx(g, s - 3 + p, w, c);
+        const int64_t h = hn + p * st;
 #pragma unroll
         for (int q = 0; q < 3; q++) A[q] = B.M.p[q1 + q][h];
         split_k_metric(RR(A[0]), RR(A[1]), RR(A[2]), sw, K);
@@ -215,7 +245,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
       code1 = entry(batch + 2 * bstep < bhi ? batch + 2 * bstep : batch + bstep);
     }
     __syncthreads();
-    const RR *const F = sF + lane;
+    const auto *const F = sF + lane;
     auto recon_p = [&](const RR *x) {
       if (!CHAR) return MET ? inner_p<SCH_HYBRID>(S, x, scm) : face_p_nonchar<SCH_HYBRID>(S, x, s, n, AXIS, scm);
       return MET ? inner_p<SCH_HYBRID>(S, x, scm) : face_p_char<SCH_HYBRID>(S, x, s, n, AXIS, scm);
@@ -259,7 +289,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
       if constexpr (MET == 2) {
         const double un = a[AXIS], ul = SL > 0 ? a[IL] : -a[IL], um = SM > 0 ? a[IM] : -a[IM];
         const double V2 = (a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) * 0.5;
-        const double KK = (gamma - 1.0) / (a[3] * a[3]);
+        const double KK = ediv(gamma - 1.0, a[3] * a[3]);
         const double KK1 = KK * 0.5;
         if (row == 0) {
           sr5[0] = 1.0 - KK * V2;
@@ -269,7 +299,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
         } else if (row < 3) {
           sr5[0] = row == 1 ? -ul : -um;
         } else {
-          const double X1 = 1.0 / (2.0 * a[3]);
+          const double X1 = ediv(1.0, 2.0 * a[3]);
           sr5[0] = row == 3 ? KK1 * V2 + X1 * un : KK1 * V2 - X1 * un;
           sr5[4] = KK1;
 #pragma unroll
@@ -287,7 +317,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
           sb5[3] = row == 1 + AXIS ? v - a[3] : v;
           sb5[4] = row == 1 + AXIS ? v + a[3] : v;
         } else {
-          const double H = V2 + 1.0 / KK;
+          const double H = V2 + ediv(1.0, KK);
           sb5[0] = V2;
           sb5[1] = ul;
           sb5[2] = um;
@@ -296,9 +326,19 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
         }
       } else {
         CharBasis Bs;
-        char_basis(gamma, a[0], a[1], a[2], a[3], a[4], a[5], a[6], Bs);
-        char_S_row(Bs, row, sr5);
-        char_S1_row(Bs, row, sb5);
+        if (row == 0) {  // needs no direction
+          Bs.u1 = a[0];
+          Bs.v1 = a[1];
+          Bs.w1 = a[2];
+          Bs.V2 = (a[0] * a[0] + a[1] * a[1] + a[2] * a[2]) * 0.5;
+          Bs.KK = ediv(gamma - 1.0, a[3] * a[3]);
+          char_S_row(Bs, 0, sr5);
+          char_S1_row(Bs, 0, sb5);
+        } else {
+          char_basis(gamma, a[0], a[1], a[2], a[3], a[4], a[5], a[6], Bs);
+          char_S_row(Bs, row, sr5);
+          char_S1_row(Bs, row, sb5);
+        }
       }
       // one flux projected (FP64) and reconstructed (RR) at a time, one
       // component's loads at a time (registers, as in the sweeps).  FP64 path:
@@ -353,7 +393,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, RR *const sFa, d
 template <int AXIS, bool CHAR, int MET, typename RR>
 __global__ __launch_bounds__(WNT) void k_weno_faces(const Block B, const int nwg) {
   // per batch:
-  __shared__ RR sF[NSUB * 80 * FB];                // [10 components][8 points][face]
+  __shared__ weno_lds_t<CHAR, RR> sF[NSUB * 80 * FB];  // [10 components][8 points][face]
   __shared__ double sQ[CHAR ? NSUB * 14 * FB : 1];  // u, v, w, c, A1..A3 at points s, s+1
   __shared__ double sG[CHAR ? NSUB * 5 * FB : 1];   // characteristic fluxes h0(1:5)
   const int wg = (int)blockIdx.x % nwg;
@@ -413,9 +453,10 @@ hipError_t weno_axis(const Block &B, hipStream_t st) {
 hipError_t launch_hybrid_lists(const Block &B, hipStream_t st) {
   const Geom &g = B.g;
   constexpr int64_t FPB = NT * LPT;
-  hipLaunchKernelGGL(k_hyb_list<0>, dim3((unsigned)((TileIndex<0>::nfaces(g) + FPB - 1) / FPB)), dim3(NT), 0, st, B);
-  hipLaunchKernelGGL(k_hyb_list<1>, dim3((unsigned)((TileIndex<1>::nfaces(g) + FPB - 1) / FPB)), dim3(NT), 0, st, B);
-  hipLaunchKernelGGL(k_hyb_list<2>, dim3((unsigned)((TileIndex<2>::nfaces(g) + FPB - 1) / FPB)), dim3(NT), 0, st, B);
+  const unsigned n0 = (unsigned)((TileIndex<0>::nfaces(g) + FPB - 1) / FPB);
+  const unsigned n1 = (unsigned)((TileIndex<1>::nfaces(g) + FPB - 1) / FPB);
+  const unsigned n2 = (unsigned)((TileIndex<2>::nfaces(g) + FPB - 1) / FPB);
+  hipLaunchKernelGGL(k_hyb_list, dim3(n0 + n1 + n2), dim3(NT), 0, st, B, n0, n1);
   return hipGetLastError();
 }
 

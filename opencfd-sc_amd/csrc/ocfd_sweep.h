@@ -312,10 +312,10 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
     }
     const R un = v[AXIS], ul = SL > 0 ? v[IL] : -v[IL], um = SM > 0 ? v[IM] : -v[IM];
     const R V2 = (v[0] * v[0] + v[1] * v[1] + v[2] * v[2]) * R(0.5);
-    const R KK = (R(gamma) - R(1.0)) / (c1 * c1);
+    const R KK = ediv(R(gamma) - R(1.0), c1 * c1);
     const R KK1 = KK * R(0.5);
-    const R X1 = R(1.0) / (R(2.0) * c1);
-    const R H = V2 + R(1.0) / KK;
+    const R X1 = ediv(R(1.0), R(2.0) * c1);
+    const R H = V2 + ediv(R(1.0), KK);
     auto dense = [&](const R *sr5) {
       R x[8];
       project(f, wl, 0, sr5, x, a1h + 3, b1h + 3);
