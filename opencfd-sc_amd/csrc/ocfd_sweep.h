@@ -36,10 +36,11 @@ __device__ constexpr inline int lidx(int m, int p, int wl) {
   return AXIS == 0 ? (m * TW + wl) * NPT + p : (m * NPT + p) * TW + wl;
 }
 
-// One tile b of a sweep of block B.  FAST != 0: the sweep axis is periodic (no
-// block-edge closures) and the metrics are uniform, both known at compile
-// time; 2: the metric vector of the axis also points along its own
-// coordinate (axis_aligned), which the projecting schemes make use of.
+// One tile b of a sweep of block B.  FAST != 0: the sweep axis is periodic, no
+// block-edge closures; 1: the metrics are uniform too; 2: and the metric
+// vector of the axis points along its own coordinate (axis_aligned), which
+// the projecting schemes make use of; 3: metric fields.  All known at compile
+// time.
 template <int AXIS, int SCH, bool CHAR, int TL, int TW, int FAST, typename R>
 __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode) {
   typedef TileIndex<AXIS> TI;
@@ -51,7 +52,8 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   static_assert(TL * TW == NTHREADS, "one cell of the tile per thread in phase 3");
   // characteristic inputs per point: u, v, w, c (+ the three normalised
   // metrics when they vary in space)
-  const bool unif = FAST || B.M.uniform != 0;
+  constexpr bool PER = FAST != 0, UNI = FAST == 1 || FAST == 2;
+  const bool unif = UNI || (FAST == 0 && B.M.uniform != 0);
   const int nq = unif ? 4 : 7;
   extern __shared__ double smem[];
 
@@ -195,8 +197,8 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
       xp[k] = q[k * PS];
       xm[k] = q[5 * CS + k * PS];
     }
-    hp = FAST ? inner_p<SCH>(S, xp, scm) : face_p_nonchar<SCH>(S, xp, s, n, AXIS, scm);
-    hm = FAST ? inner_m<SCH>(S, xm, scm) : face_m_nonchar<SCH>(S, xm, s, n, AXIS, scm);
+    hp = PER ? inner_p<SCH>(S, xp, scm) : face_p_nonchar<SCH>(S, xp, s, n, AXIS, scm);
+    hm = PER ? inner_m<SCH>(S, xm, scm) : face_m_nonchar<SCH>(S, xm, s, n, AXIS, scm);
   };
   // (fs: the face's first stencil point)
 // after a characteristic row: the next one reads its stencil again (kept in
@@ -262,10 +264,10 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
     char_S_row(Bs, r, sr5);
     // outside the scheme's stencil the projected value is 0
     project(f, wl, 0, sr5, x, a1h + 3, b1h + 3);
-    const R h1 = FAST ? inner_p<SCH>(S, x, scm) : face_p_char<SCH>(S, x, s, n, AXIS, scm);
+    const R h1 = PER ? inner_p<SCH>(S, x, scm) : face_p_char<SCH>(S, x, s, n, AXIS, scm);
     __builtin_amdgcn_sched_barrier(0);
     project(f, wl, 5, sr5, x, a2h + 3, b2h + 3);
-    const R h2 = FAST ? inner_m<SCH>(S, x, scm) : face_m_char<SCH>(S, x, s, n, AXIS, scm);
+    const R h2 = PER ? inner_m<SCH>(S, x, scm) : face_m_char<SCH>(S, x, s, n, AXIS, scm);
     return h1 + h2;
   };
   // component m of a linear (hybrid UD7L) face: no projection
@@ -274,8 +276,8 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
     R xp[8], xm[8];
 #pragma unroll
     for (int k = 0; k < 8; k++) { xp[k] = FPV(m, k); xm[k] = FMV(m, k); }
-    const R h1 = FAST ? inner_p<SCH>(S, xp, 1) : face_p_char<SCH>(S, xp, s, n, AXIS, 1);
-    const R h2 = FAST ? inner_m<SCH>(S, xm, 1) : face_m_char<SCH>(S, xm, s, n, AXIS, 1);
+    const R h1 = PER ? inner_p<SCH>(S, xp, 1) : face_p_char<SCH>(S, xp, s, n, AXIS, 1);
+    const R h2 = PER ? inner_m<SCH>(S, xm, 1) : face_m_char<SCH>(S, xm, s, n, AXIS, 1);
     return h1 + h2;
   };
   // non-reflecting closure of component m (OCFD_inviscous_character.f90:295-309);
@@ -401,7 +403,7 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   auto item_ch = [&](int it, int &f, int &wl) {
     if (AXIS == 0) { f = it % NF; wl = it / NF; } else { wl = it % TW; f = it / TW; }
   };
-  const bool closure_lo = !FAST && lo == 1 && sl == 0, closure_hi = !FAST && hi == 1 && sr == 0;
+  const bool closure_lo = !PER && lo == 1 && sl == 0, closure_hi = !PER && hi == 1 && sr == 0;
   auto slot_of = [&](int f, int wl) { return sS[lidx<AXIS, NF, TW>(0, f, wl)]; };
   // work items of this thread: (component, face, line), or on the
   // characteristic path (face, line) with all five components, so that the
@@ -631,7 +633,7 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
       *dst = pdu[m] + val;
     } else {
       const int64_t h = TI::hidx(g, s0 + c3s, w0 + c3w, c);
-      R rr = -(pdu[m] + val) * R(FAST ? B.M.u[M_AJAC] : B.M.get(M_AJAC, h));
+      R rr = -(pdu[m] + val) * R(UNI ? B.M.u[M_AJAC] : (FAST == 3 ? B.M.p[M_AJAC][h] : B.M.get(M_AJAC, h)));
       if (B.P.if_mass_force == 1 && m > 0) {
         // OCFD_inviscous.f90:189-201
         const double *mf = B.P.mass_force;
@@ -703,7 +705,7 @@ hipError_t dispatch_scheme(const Block &B, int mode, hipStream_t st) {
     case SCH_OMP6: return launch_one<AXIS, SCH_OMP6, CHAR, TL, TW, FAST, R>(B, mode, st);
     case SCH_UD7L: return launch_one<AXIS, SCH_UD7L, CHAR, TL, TW, FAST, R>(B, mode, st);
     // (its faces are not projected in the sweep)
-    case SCH_HYBRID: return launch_one<AXIS, SCH_HYBRID, CHAR, TL, TW, FAST ? 1 : 0, R>(B, mode, st);
+    case SCH_HYBRID: return launch_one<AXIS, SCH_HYBRID, CHAR, TL, TW, FAST == 2 ? 1 : FAST, R>(B, mode, st);
     default: return hipErrorInvalidValue;
   }
 }
@@ -768,7 +770,17 @@ hipError_t dispatch_axis(const Block &B, int mode, int shape, hipStream_t st) {
       return ch ? dispatch_scheme<AXIS, true, 2, R, 2>(B, mode, st) : dispatch_scheme<AXIS, false, 1, R, 2>(B, mode, st);
     return ch ? dispatch_scheme<AXIS, true, 2, R, 0>(B, mode, st) : dispatch_scheme<AXIS, false, 1, R, 0>(B, mode, st);
   }
-  if (general_shape<AXIS>(B.g) == 1)
+  // metric fields: a periodic axis without the block-edge closures (whose
+  // branches cost a tenth of a sweep's instructions: hybrid 160^3 in FP64, x,
+  // y, z 140, 175, 201 -> 116, 157, 190 us; z of 240 x 100 x 48, WENO5 char,
+  // 121 -> 115)
+  const int gshape = general_shape<AXIS>(B.g);
+  if (B.S.iperiodic[AXIS] == 1) {
+    if (gshape == 1)
+      return ch ? dispatch_scheme<AXIS, true, 3, R, 1>(B, mode, st) : dispatch_scheme<AXIS, false, 3, R, 1>(B, mode, st);
+    return ch ? dispatch_scheme<AXIS, true, 3, R, 0>(B, mode, st) : dispatch_scheme<AXIS, false, 3, R, 0>(B, mode, st);
+  }
+  if (gshape == 1)
     return ch ? dispatch_scheme<AXIS, true, 0, R, 1>(B, mode, st) : dispatch_scheme<AXIS, false, 0, R, 1>(B, mode, st);
   return ch ? dispatch_scheme<AXIS, true, 0, R, 0>(B, mode, st) : dispatch_scheme<AXIS, false, 0, R, 0>(B, mode, st);
 }
