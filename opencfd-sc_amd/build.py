@@ -24,7 +24,8 @@ LIB = os.path.join(HERE, "libocfd_hip.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
-SOURCES = ["ocfd_inviscid.hip", "ocfd_inviscid_mixed.hip", "ocfd_hybrid.hip", "ocfd_viscous.hip",
+SOURCES = ["ocfd_inviscid.hip", "ocfd_inviscid_mixed.hip", "ocfd_inviscid_xyz.hip", "ocfd_inviscid_xyz_mixed.hip",
+           "ocfd_hybrid.hip", "ocfd_viscous.hip",
            "ocfd_viscous_mixed.hip", "ocfd_misc.hip", "ocfd_batchq.hip", "ocfd_batchq_mixed.hip",
            "ocfd_api.hip"]
 

@@ -73,6 +73,10 @@ struct ocfd_handle {
   // stage is all that writes halos, so it writes both buffers of T (u, v, w)
   // and the repair copies none (mixed 256^3: repair 61 -> 4 us per stage)
   bool halo_both = false;
+  // small blocks: the y and z parts of du of whole steps, whose three sweeps
+  // are one launch (k_inviscid_xyz); NULL where the sweeps run one by one
+  double *du_yz = nullptr;
+  bool du_parts = false;  // du holds the x part alone (settle_du joins them)
   // per-routine calls merged into the whole-step stage kernels
   // (ocfd_set_stage_fusion); pend holds what the stage so far left to do
   bool stage_fusion = false;
@@ -279,6 +283,18 @@ __global__ void k_patch(const Geom g, double *r, int ib, int ie, int jb, int je,
   r[q] = r[q] + 100.0;
 }
 
+// Whole steps of blocks up to this size run their three sweeps in one launch
+// (k_inviscid_xyz).  A sweep of a small block does not fill the chip and its
+// launch costs as much as its arithmetic; of a larger one the launches are a
+// few percent, and the two more arrays that the stage update reads cost more
+// than they save.  Step times, three launches and one, us: WENO5 32^3 130 and
+// 95, 64^3 291 and 265, 96^3 780 and 742; WENO7 characteristic 32^3 183 and
+// 122, 80^3 815 and 760, 96^3 1172 and 1180, 104^3 1565 and 1611; hybrid, tuned
+// tiles, 80^3 1078 and 1054, 96^3 1728 and 1733, 112^3 2077 and 2151; in mixed
+// precision 80^3 704 and 675, 104^3 1238 and 1241; WENO5 characteristic plate
+// 120 x 100 x 48 1206 and 1180, 200 x 100 x 40 1608 and 1610.
+constexpr int64_t XYZ_MAX_CELLS = 600000;
+
 int alloc(double **p, size_t bytes) {
   if (hipMalloc((void **)p, bytes) != hipSuccess) {
     *p = nullptr;
@@ -380,7 +396,22 @@ int upload_prims(ocfd_handle *h, const double *const src[5], bool make_f) {
   return rc;
 }
 
-int inviscid(ocfd_handle *h, bool ch) {
+// a block whose right-hand side is in the three sweeps' parts
+Block with_parts(const ocfd_handle *h, Block B) {
+  B.du2 = h->du_yz;
+  B.du3 = h->du_yz + 5 * B.g.ni;
+  return B;
+}
+// du as the z sweep leaves it, for its readers outside whole steps
+int settle_du(ocfd_handle *h) {
+  if (!h->du_parts) return 0;
+  h->du_parts = false;
+  return launch(h, "du_join", [&] { return launch_du_join(with_parts(h, h->B), h->st); });
+}
+
+// xyz: the three sweeps in one launch into the parts of du (whole steps of
+// small blocks, ocfd_handle::du_yz)
+int inviscid(ocfd_handle *h, bool ch, bool xyz = false) {
   Block B = h->B;
   B.S.is_char = ch ? 1 : 0;
   if (B.hcount) {
@@ -389,6 +420,8 @@ int inviscid(ocfd_handle *h, bool ch) {
       return fail("hybrid scheme: the inviscid routine must match IF_Scheme_Character");
     if (launch(h, "weno_faces", [&] { return launch_weno_faces(B, h->st); })) return -1;
   }
+  h->du_parts = xyz;
+  if (xyz) return launch(h, "inviscid_xyz", [&] { return launch_inviscid_xyz(with_parts(h, B), h->st); });
   static const char *nm[2][3] = {{"inviscid_x", "inviscid_y", "inviscid_z"},
                                  {"inviscid_char_x", "inviscid_char_y", "inviscid_char_z"}};
   const int modes[3] = {INV_ASSIGN, INV_ACCUM, INV_FINAL};
@@ -532,7 +565,14 @@ int ocfd_create(const ocfd_config *cfg, int device, ocfd_handle **out) {
   if (h->fused)
     for (PrimField *p : {&B.u2, &B.v2, &B.w2}) rc |= alloc_prim(p, B.g.nh, p32);
   B.halt = nullptr;
+  B.du2 = B.du3 = nullptr;
   rc |= alloc(&B.f, fb) | alloc(&B.fn, fb) | alloc(&B.du, fb);
+  // without room for it the sweeps run one by one
+  // (the mass force is added by the z sweep)
+  if (B.g.ni <= XYZ_MAX_CELLS && cfg->if_mass_force != 1 && hipMalloc((void **)&h->du_yz, 2 * fb) != hipSuccess) {
+    h->du_yz = nullptr;
+    (void)hipGetLastError();
+  }
   if (cfg->scheme_invis == SCH_HYBRID) rc |= alloc(&B.rhyb, hb);
   if (cfg->if_viscous == 1) rc |= alloc(&B.ev, 12 * (size_t)B.g.ni * sizeof(double));
   if (cfg->nfiltering > 0) rc |= alloc(&h->fbuf, fb);
@@ -613,7 +653,7 @@ int ocfd_destroy(ocfd_handle *h) {
   Block &B = h->B;
   for (const PrimField *p : {&B.d, &B.u, &B.v, &B.w, &B.T, &B.T2, &B.u2, &B.v2, &B.w2})
     if (p->p) (void)hipFree(p->p);
-  double *ps[] = {B.f, B.fn, B.du, B.rhyb, B.ev, h->fbuf, h->work, h->wout};
+  double *ps[] = {B.f, B.fn, B.du, h->du_yz, B.rhyb, B.ev, h->fbuf, h->work, h->wout};
   for (double *p : ps)
     if (p) (void)hipFree(p);
   for (int a = 0; a < 3; a++) {
@@ -643,6 +683,7 @@ int ocfd_synchronize(ocfd_handle *h) {
 // ---- grid / metrics --------------------------------------------------------
 int ocfd_set_grid(ocfd_handle *h, const double *x, const double *y, const double *z, const double spans[9]) {
   if (h->B.M.uniform) return fail("ocfd_set_grid needs OCFD_METRIC_FIELD");
+  if (settle_du(h)) return -1;
   const Geom &g = h->B.g;
   std::vector<double> stage((size_t)g.nh);
   double *dc[3] = {};
@@ -669,12 +710,17 @@ int ocfd_set_grid(ocfd_handle *h, const double *x, const double *y, const double
 
 int ocfd_upload_metrics(ocfd_handle *h, const double *const metrics[19]) {
   if (h->B.M.uniform) return fail("ocfd_upload_metrics needs OCFD_METRIC_FIELD");
+  if (h->du_parts) {
+    if (settle_du(h)) return -1;
+    HIPCHK(hipStreamSynchronize(h->st));
+  }
   for (int m = 0; m < M_N; m++) HIPCHK(hipMemcpy(h->met[m], metrics[m], h->halo_bytes(), hipMemcpyHostToDevice));
   return 0;
 }
 
 int ocfd_set_uniform_metrics(ocfd_handle *h, const double m[10]) {
   if (!h->B.M.uniform) return fail("ocfd_set_uniform_metrics needs OCFD_METRIC_UNIFORM");
+  if (settle_du(h)) return -1;
   for (int q = 0; q < 10; q++) h->B.M.u[q] = m[q];
   for (int q = 0; q < 9; q++) h->B.M.u[M_AKX1 + q] = m[q] / m[M_AJAC];
   set_split_const(h->B);
@@ -830,6 +876,7 @@ int ocfd_download_fn(ocfd_handle *h, double *f) {
 }
 // du is FP32 on the device in the mixed-precision form: converted on the host
 int ocfd_download_du(ocfd_handle *h, double *f) {
+  if (settle_du(h)) return -1;
   HIPCHK(hipStreamSynchronize(h->st));
   if (h->B.prec != OCFD_PREC_MIXED_CODE) {
     HIPCHK(hipMemcpy(f, h->B.du, h->f_bytes(), hipMemcpyDeviceToHost));
@@ -842,6 +889,7 @@ int ocfd_download_du(ocfd_handle *h, double *f) {
   return 0;
 }
 int ocfd_upload_du(ocfd_handle *h, const double *f) {
+  h->du_parts = false;
   if (h->B.prec != OCFD_PREC_MIXED_CODE) {
     HIPCHK(hipMemcpy(h->B.du, f, h->f_bytes(), hipMemcpyHostToDevice));
     return 0;
@@ -901,6 +949,7 @@ int ocfd_du_inviscous_character(ocfd_handle *h) { return inviscid(h, true); }
 
 int ocfd_du_viscous(ocfd_handle *h) {
   if (!h->B.ev) return fail("du_viscous needs IF_Viscous = 1");
+  if (settle_du(h)) return -1;
   if (h->stage_fusion) {
     // the fluxes now (inside the update for a fused block); their
     // divergence joins the update in ocfd_time_adv_rk3
@@ -914,6 +963,7 @@ int ocfd_du_viscous(ocfd_handle *h) {
 
 int ocfd_time_adv_rk3(ocfd_handle *h, int32_t krk) {
   if (krk < 1 || krk > 3) return fail("KRK must be 1, 2 or 3");
+  if (settle_du(h)) return -1;
   if (h->stage_fusion) {
     // ocfd_step's stage update: viscous divergence (when du_viscous ran),
     // RK3 (fn = f at KRK = 1), primitives, boundary-plane f on periodic
@@ -1095,16 +1145,17 @@ int step_body(ocfd_handle *h) {
   for (int krk = 1; krk <= 3; krk++) {
     if (h->halo_both ? exchange_stage(h) : exchange_prims(h)) return -1;
     if (krk == 1 && hyb && sensor(h)) return -1;
-    if (inviscid(h, ch)) return -1;
+    const bool xyz = h->du_yz != nullptr;
+    if (inviscid(h, ch, xyz)) return -1;
     const int refresh = h->ibc == 0 ? 1 : 0;
+    Block B = xyz ? with_parts(h, h->B) : h->B;
     if (h->fused) {
       // viscous terms, divergence and update in one march (k_visc_fused)
-      if (launch(h, "stage_update_fused", [&] { return launch_visc_fused(h->B, krk, refresh, h->neg, h->st); }))
+      if (launch(h, "stage_update_fused", [&] { return launch_visc_fused(B, krk, refresh, h->neg, h->st); }))
         return -1;
       swap_uvw(h);
     } else {
       if (c.if_viscous == 1 && launch(h, "visc_flux", [&] { return launch_visc_flux(h->B, h->st); })) return -1;
-      Block B = h->B;
       if (c.if_viscous != 1) B.ev = nullptr;
       if (launch(h, "stage_update", [&] { return launch_visc_div_update(B, krk, refresh, h->neg, h->st); }))
         return -1;
@@ -1178,6 +1229,7 @@ int ocfd_step(ocfd_handle *h, int32_t nsteps) {
         if (h->fused) swap_uvw(h);
       }
       if (!rc && hipGraphLaunch(h->gexec[p], h->st) != hipSuccess) rc = fail("hipGraphLaunch failed");
+      h->du_parts = h->du_yz != nullptr;
     } else {
       rc = step_body(h);
     }
@@ -1240,6 +1292,7 @@ int ocfd_autotune(ocfd_handle *h, int32_t reps, int32_t shape_out[3]) {
   if (rc) return -1;
   Block B = h->B;
   B.S.is_char = ch ? 1 : 0;
+  h->du_parts = false;
   const int modes[3] = {INV_ASSIGN, INV_ACCUM, INV_FINAL};
   hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
@@ -1808,6 +1861,7 @@ int ocfd_batch_step(ocfd_batch *b, int32_t nsteps) {
   std::vector<int> istep0(nbox);
   std::vector<double> tt0(nbox);
   for (int i = 0; i < nbox; i++) {
+    b->box[i]->du_parts = false;  // the batch's sweeps write du itself
     istep0[i] = b->box[i]->istep;
     tt0[i] = b->box[i]->tt;
   }

@@ -49,7 +49,7 @@ __device__ __forceinline__ void q_sweep_scheme(const Block &B, int lt, int mode)
     else march_tile<AXIS, SCH, false, R>(B, lt, mode, SL);
   } else {
     constexpr int TL = shape_tl<AXIS>(SHAPE), TW = NTHREADS / TL;
-    sweep_tile<AXIS, SCH, false, TL, TW, true, R>(B, lt, mode);
+    sweep_tile<AXIS, SCH, false, TL, TW, 1, R>(B, lt, mode, B.du);
   }
 }
 
@@ -147,8 +147,8 @@ void k_batch_queue(const QPlan P) {
         const Block B = S.blk[box];
         int *neg = P.neg + NEG_STRIDE * box;
         const int ks = batch_kseg_dev(B);
-        if (sg.visc) visc_div_update_tile<true, false, true, R>(B, stage, 1, ks, neg, lt);
-        else visc_div_update_tile<false, false, true, R>(B, stage, 1, ks, neg, lt);
+        if (sg.visc) visc_div_update_tile<true, false, true, R, false>(B, stage, 1, ks, neg, lt);
+        else visc_div_update_tile<false, false, true, R, false>(B, stage, 1, ks, neg, lt);
         break;
       }
       default: {  // Q_REPAIR: item 0 of a box repairs, the others copy T's halo into T2

@@ -55,6 +55,9 @@ struct Block {
   // stage-start ones, and the host swaps the sets after every fused stage.
   PrimField u2, v2, w2;
   double *f, *fn, *du;        // 5 planes each
+  // whole steps of small blocks (NULL elsewhere): the y and z sweeps' parts of
+  // du, beside the x sweep's in du; the stage update adds them (tri_du)
+  double *du2, *du3;
   double *rhyb;               // halo'd sensor (hybrid scheme only)
   double *ev;                 // 12 interior planes: Ev1(1:4), Ev2(1:4), Ev3(1:4)
   // hybrid scheme, per sweep axis: the faces that use WENO7/WENO5 (face id
@@ -100,6 +103,12 @@ inline bool prims_match(const Block &B) {
   return B.d.f32 == f32 && B.u.f32 == f32 && B.v.f32 == f32 && B.w.f32 == f32 && B.T.f32 == f32 &&
          B.T2.f32 == f32 && (!B.u2.p || B.u2.f32 == f32) && (!B.v2.p || B.v2.f32 == f32) &&
          (!B.w2.p || B.w2.f32 == f32);
+}
+// du from the three sweeps' parts x, y, z: the sum and the factor -Ajac of the
+// z sweep's last step (sweep_tile, mode INV_FINAL), in the same order and type
+template <typename RT>
+__device__ inline RT tri_du(const RT x, const RT y, const RT z, const RT ajac) {
+  return -((x + y) + z) * ajac;
 }
 __device__ inline bool halted(const Block &B) { return B.halt != nullptr && *B.halt != 0; }
 
@@ -272,6 +281,10 @@ struct BLArgs {
 
 // ---- launchers (return hipError_t of the launch) ----
 hipError_t launch_inviscid(const Block &B, int axis, int mode, SweepTile tile, hipStream_t st);
+// the three sweeps in one launch, into du, du2 and du3 (no mass force);
+// their join in du
+hipError_t launch_inviscid_xyz(const Block &B, hipStream_t st);
+hipError_t launch_du_join(const Block &B, hipStream_t st);
 hipError_t launch_hybrid_lists(const Block &B, hipStream_t st);
 // batched launches over the boxes of S (ntiles workgroups in all)
 hipError_t launch_inviscid_batch(const BoxSet &S, int prec, int axis, int sch, bool ch, int mode, int shape,

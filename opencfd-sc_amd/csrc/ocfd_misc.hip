@@ -209,6 +209,19 @@ __global__ __launch_bounds__(NT) void k_rk3(const Block B, const int krk) {
   }
 }
 
+// du from the three sweeps' parts (tri_du), one component per blockIdx.y
+template <typename DU>
+__global__ __launch_bounds__(NT) void k_du_join(const Block B) {
+  const Geom &g = B.g;
+  const int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
+  if (t >= g.ni) return;
+  const int i = (int)(t % g.nx) + 1, j = (int)(t / g.nx % g.ny) + 1, k = (int)(t / ((int64_t)g.nx * g.ny)) + 1;
+  const int64_t q = t + blockIdx.y * g.ni;
+  DU *const x = reinterpret_cast<DU *>(B.du);
+  x[q] = tri_du(x[q], reinterpret_cast<const DU *>(B.du2)[q], reinterpret_cast<const DU *>(B.du3)[q],
+                DU(B.M.get(M_AJAC, g.hi(i, j, k))));
+}
+
 __global__ __launch_bounds__(NT) void k_copy(const double *src, double *dst, int64_t n) {
   const int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
   if (t < n) dst[t] = src[t];
@@ -913,6 +926,13 @@ hipError_t launch_hybrid_counts(const Block &B, unsigned long long *counts, hipS
 hipError_t launch_rk3(const Block &B, int krk, hipStream_t st) {
   if (B.prec == OCFD_PREC_MIXED_CODE) hipLaunchKernelGGL(k_rk3<float>, dim3(nb(5 * B.g.ni)), dim3(NT), 0, st, B, krk);
   else hipLaunchKernelGGL(k_rk3<double>, dim3(nb(5 * B.g.ni)), dim3(NT), 0, st, B, krk);
+  return hipGetLastError();
+}
+
+hipError_t launch_du_join(const Block &B, hipStream_t st) {
+  const dim3 grid(nb(B.g.ni), 5);
+  if (B.prec == OCFD_PREC_MIXED_CODE) hipLaunchKernelGGL(k_du_join<float>, grid, dim3(NT), 0, st, B);
+  else hipLaunchKernelGGL(k_du_join<double>, grid, dim3(NT), 0, st, B);
   return hipGetLastError();
 }
 

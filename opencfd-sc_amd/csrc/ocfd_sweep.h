@@ -42,7 +42,7 @@ __device__ constexpr inline int lidx(int m, int p, int wl) {
 // the projecting schemes make use of; 3: metric fields.  All known at compile
 // time.
 template <int AXIS, int SCH, bool CHAR, int TL, int TW, int FAST, typename R>
-__device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode) {
+__device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode, double *const du_out) {
   typedef TileIndex<AXIS> TI;
   constexpr int NP = TL + 8;  // points s0-4 .. s0+TL+3
   constexpr int NF = TL + 1;  // faces  s0-1 .. s0+TL-1
@@ -102,7 +102,7 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   // du entries of the tile (accumulating modes), fetched before the face
   // fluxes are computed
   // du is stored in the sweep's real type (FP32 in the mixed-precision form)
-  R *const du = reinterpret_cast<R *>(B.du);
+  R *const du = reinterpret_cast<R *>(du_out);
   R pdu[5];
   const int64_t c3i = TI::iidx(g, s0 + c3s, w0 + c3w, c);
 
@@ -648,7 +648,7 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
 // one block: the tiles in XCD order
 template <int AXIS, int SCH, bool CHAR, int TL, int TW, int FAST, typename R>
 __global__ __launch_bounds__(NTHREADS) void k_inviscid(const Block B, const int mode) {
-  sweep_tile<AXIS, SCH, CHAR, TL, TW, FAST, R>(B, xcd_tile(blockIdx.x, gridDim.x), mode);
+  sweep_tile<AXIS, SCH, CHAR, TL, TW, FAST, R>(B, xcd_tile(blockIdx.x, gridDim.x), mode, B.du);
 }
 
 // a batch of periodic boxes with uniform metrics: the tiles of all boxes of
@@ -659,7 +659,8 @@ __global__ __launch_bounds__(NTHREADS) void k_inviscid_batch(const BoxSet S, con
   const int j = S.entry(t);
   // the descriptor is read in place (a local copy would live in scratch:
   // the sweep indexes some of its arrays at run time)
-  sweep_tile<AXIS, SCH, CHAR, TL, TW, 1, R>(S.blk[S.ids[j]], t - S.off[j], mode);
+  const Block &B = S.blk[S.ids[j]];
+  sweep_tile<AXIS, SCH, CHAR, TL, TW, 1, R>(B, t - S.off[j], mode, B.du);
 }
 
 // LDS bytes of a sweep tile: split fluxes, characteristic inputs, face fluxes
@@ -792,6 +793,66 @@ hipError_t launch_sweep(const Block &B, int axis, int mode, int shape, hipStream
   if (axis == 0) return dispatch_axis<0, R>(B, mode, shape, st);
   if (axis == 1) return dispatch_axis<1, R>(B, mode, shape, st);
   return dispatch_axis<2, R>(B, mode, shape, st);
+}
+
+// ---- the three sweeps of a small block in one launch -----------------------
+// A sweep of a block of up to a few 10^5 cells is a chain of latencies -- two
+// rounds of loads, the rounds of faces of a tile, the store -- on a chip it
+// does not fill, and its three sweeps are independent but for the sum in du.
+// One launch runs the tiles of all three axes, each into its own array (B.du,
+// B.du2, B.du3), and the stage update adds them as the sweeps would have
+// (tri_du).  Shape 1: the more and smaller tiles.  WENO5 32^3, x, y and z: 25
+// us in three launches, 12 in one.
+template <int SCH, bool CHAR, int FAST, typename R>
+__global__ __launch_bounds__(NTHREADS) void k_inviscid_xyz(const Block B, const int n0, const int n1) {
+  const int b = (int)blockIdx.x;
+  if (b < n0)
+    sweep_tile<0, SCH, CHAR, shape_tl<0>(1), NTHREADS / shape_tl<0>(1), FAST, R>(B, xcd_tile(b, n0), INV_ASSIGN, B.du);
+  else if (b < n0 + n1)
+    sweep_tile<1, SCH, CHAR, shape_tl<1>(1), NTHREADS / shape_tl<1>(1), FAST, R>(B, xcd_tile(b - n0, n1), INV_ASSIGN,
+                                                                                 B.du2);
+  else
+    sweep_tile<2, SCH, CHAR, shape_tl<2>(1), NTHREADS / shape_tl<2>(1), FAST, R>(
+        B, xcd_tile(b - n0 - n1, (int)gridDim.x - n0 - n1), INV_ASSIGN, B.du3);
+}
+
+template <int SCH, bool CHAR, int FAST, typename R>
+hipError_t launch_xyz_one(const Block &B, hipStream_t st) {
+  constexpr bool HYB = (SCH == SCH_HYBRID);
+  const int nq = B.M.uniform ? 4 : 7;
+  const size_t lx = sweep_lds<shape_tl<0>(1), NTHREADS / shape_tl<0>(1), CHAR, HYB, R>(nq);
+  const size_t ly = sweep_lds<shape_tl<1>(1), NTHREADS / shape_tl<1>(1), CHAR, HYB, R>(nq);
+  const int n0 = (int)sweep_tiles(B.g, 0, 1), n1 = (int)sweep_tiles(B.g, 1, 1), n2 = (int)sweep_tiles(B.g, 2, 1);
+  hipLaunchKernelGGL((k_inviscid_xyz<SCH, CHAR, FAST, R>), dim3((unsigned)(n0 + n1 + n2)), dim3(NTHREADS),
+                     lx > ly ? lx : ly, st, B, n0, n1);
+  return hipGetLastError();
+}
+
+template <bool CHAR, int FAST, typename R>
+hipError_t dispatch_xyz(const Block &B, hipStream_t st) {
+  switch (B.S.scheme_invis) {
+    case SCH_WENO5: return launch_xyz_one<SCH_WENO5, CHAR, FAST, R>(B, st);
+    case SCH_WENO7: return launch_xyz_one<SCH_WENO7, CHAR, FAST, R>(B, st);
+    case SCH_OMP6: return launch_xyz_one<SCH_OMP6, CHAR, FAST, R>(B, st);
+    case SCH_UD7L: return launch_xyz_one<SCH_UD7L, CHAR, FAST, R>(B, st);
+    case SCH_HYBRID: return launch_xyz_one<SCH_HYBRID, CHAR, FAST == 2 ? 1 : FAST, R>(B, st);
+    default: return hipErrorInvalidValue;
+  }
+}
+
+// periodic uniform grids (for the projecting schemes: metric vectors along
+// their coordinates), periodic metric fields, or the general kernel
+template <typename R>
+hipError_t launch_sweep_xyz(const Block &B, hipStream_t st) {
+  const bool ch = B.S.is_char != 0;
+  const bool per = B.S.iperiodic[0] == 1 && B.S.iperiodic[1] == 1 && B.S.iperiodic[2] == 1;
+  if (per && B.M.uniform) {
+    if (!ch) return dispatch_xyz<false, 1, R>(B, st);
+    if (B.S.scheme_invis == SCH_HYBRID || (axis_aligned<0>(B.M) && axis_aligned<1>(B.M) && axis_aligned<2>(B.M)))
+      return dispatch_xyz<true, 2, R>(B, st);
+  }
+  if (per && !B.M.uniform) return ch ? dispatch_xyz<true, 3, R>(B, st) : dispatch_xyz<false, 3, R>(B, st);
+  return ch ? dispatch_xyz<true, 0, R>(B, st) : dispatch_xyz<false, 0, R>(B, st);
 }
 
 // ---- batches (ocfd_batch): periodic boxes with uniform metrics, no hybrid --

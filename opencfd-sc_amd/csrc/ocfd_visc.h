@@ -318,7 +318,9 @@ __device__ inline void refresh_of(double cv, double d, double u, double v, doubl
 // one wave per SIMD (its register footprint), so the loads of plane k+1 --
 // du, f, fn of the own cell and the Ev tiles -- are all issued at the top of
 // iteration k to keep enough bytes in flight.
-template <bool VISC, bool CD8, bool FAST, typename RT>
+// TRI: du is in the three sweeps' parts (tri_du), loaded in the iteration that
+// uses them.
+template <bool VISC, bool CD8, bool FAST, typename RT, bool TRI>
 __device__ __forceinline__ void visc_div_update_tile(const Block &B, const int krk, const int refresh, const int kseg,
                                                      int *neg, const int tile) {
   typedef PlaneTile<CD8> PT;
@@ -429,7 +431,7 @@ __device__ __forceinline__ void visc_div_update_tile(const Block &B, const int k
     const int64_t t = col + (int64_t)(k - 1) * skz;
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-      c.du[m] = double(__builtin_nontemporal_load(&dus[t + m * ni]));
+      c.du[m] = TRI ? 0.0 : double(__builtin_nontemporal_load(&dus[t + m * ni]));
       c.f[m] = __builtin_nontemporal_load(&B.f[t + m * ni]);
       c.fn[m] = krk != 1 ? __builtin_nontemporal_load(&B.fn[t + m * ni]) : 0.0;
     }
@@ -446,6 +448,14 @@ __device__ __forceinline__ void visc_div_update_tile(const Block &B, const int k
     const int kn = k < tc.ke ? k + 1 : k;
     const CellVals cn = fetch_cell(kn);
     const double *du = cv.du, *f0 = cv.f, *fn0 = cv.fn;
+    RT part[3][TRI ? 5 : 1];
+    if constexpr (TRI) {
+      const RT *const q[3] = {dus, reinterpret_cast<const RT *>(B.du2), reinterpret_cast<const RT *>(B.du3)};
+#pragma unroll
+      for (int a = 0; a < 3; a++)
+#pragma unroll
+        for (int m = 0; m < 5; m++) part[a][m] = q[a][t + m * ni];
+    }
     RT qn[4];
     if (VISC) {
       fetch_tile(kn);
@@ -471,7 +481,9 @@ __device__ __forceinline__ void visc_div_update_tile(const Block &B, const int k
     double fq[5];
 #pragma unroll
     for (int m = 0; m < 5; m++) {
-      double dum = du[m];
+      double dum;
+      if constexpr (TRI) dum = double(tri_du(part[0][m], part[1][m], part[2][m], RT(ajac)));
+      else dum = du[m];
       if (VISC && m > 0) dum = dum + double(vd[m]) * ajac;
       const double f = f0[m];
       double r;
@@ -523,10 +535,10 @@ __device__ __forceinline__ void visc_div_update_tile(const Block &B, const int k
   }
 }
 
-template <bool VISC, bool CD8, bool FAST, typename RT>
+template <bool VISC, bool CD8, bool FAST, typename RT, bool TRI>
 __global__ __launch_bounds__(NT) void k_visc_div_update(const Block B, const int krk, const int refresh,
                                                         const int kseg, int *neg) {
-  visc_div_update_tile<VISC, CD8, FAST, RT>(B, krk, refresh, kseg, neg, xcd_tile(blockIdx.x, gridDim.x));
+  visc_div_update_tile<VISC, CD8, FAST, RT, TRI>(B, krk, refresh, kseg, neg, xcd_tile(blockIdx.x, gridDim.x));
 }
 
 // Batches of periodic boxes with uniform metrics (ocfd_batch): the tiles of
@@ -550,7 +562,7 @@ __global__ __launch_bounds__(NT) void k_visc_div_update_batch(const BoxSet S, co
   const int j = S.entry(t);
   const int box = S.ids[j];
   const Block B = S.blk[box];  // copied before any store, as above
-  visc_div_update_tile<VISC, CD8, true, RT>(B, krk, 1, batch_kseg_dev(B), neg + NEG_STRIDE * box, t - S.off[j]);
+  visc_div_update_tile<VISC, CD8, true, RT, false>(B, krk, 1, batch_kseg_dev(B), neg + NEG_STRIDE * box, t - S.off[j]);
 }
 
 // ---------------------------------------------------------------------------
@@ -633,23 +645,28 @@ hipError_t visc_div_as(const Block &B, hipStream_t st) {
   return hipGetLastError();
 }
 
-template <bool VISC, bool CD8, bool FAST, typename RT>
+template <bool VISC, bool CD8, bool FAST, typename RT, bool TRI>
 void launch_update_one(const Block &B, int krk, int refresh_planes, int *neg, hipStream_t st) {
   static int cache[64] = {};
   const int kseg =
-      march_kseg(B.g, resident_groups(k_visc_div_update<VISC, CD8, FAST, RT>, cache), march_kmax<RT>());
-  hipLaunchKernelGGL((k_visc_div_update<VISC, CD8, FAST, RT>), dim3(march_blocks(B.g, kseg)), dim3(NT), 0, st, B, krk,
-                     refresh_planes, kseg, neg);
+      march_kseg(B.g, resident_groups(k_visc_div_update<VISC, CD8, FAST, RT, TRI>, cache), march_kmax<RT>());
+  hipLaunchKernelGGL((k_visc_div_update<VISC, CD8, FAST, RT, TRI>), dim3(march_blocks(B.g, kseg)), dim3(NT), 0, st, B,
+                     krk, refresh_planes, kseg, neg);
+}
+template <typename RT, bool TRI>
+hipError_t visc_div_update_of(const Block &B, int krk, int refresh_planes, int *neg, hipStream_t st) {
+  const bool cd8 = B.S.scheme_vis == SCH_CD8, per = all_periodic(B);
+  if (B.ev == nullptr) launch_update_one<false, false, false, RT, TRI>(B, krk, refresh_planes, neg, st);
+  else if (cd8 && per) launch_update_one<true, true, true, RT, TRI>(B, krk, refresh_planes, neg, st);
+  else if (cd8) launch_update_one<true, true, false, RT, TRI>(B, krk, refresh_planes, neg, st);
+  else if (per) launch_update_one<true, false, true, RT, TRI>(B, krk, refresh_planes, neg, st);
+  else launch_update_one<true, false, false, RT, TRI>(B, krk, refresh_planes, neg, st);
+  return hipGetLastError();
 }
 template <typename RT>
 hipError_t visc_div_update_as(const Block &B, int krk, int refresh_planes, int *neg, hipStream_t st) {
-  const bool cd8 = B.S.scheme_vis == SCH_CD8, per = all_periodic(B);
-  if (B.ev == nullptr) launch_update_one<false, false, false, RT>(B, krk, refresh_planes, neg, st);
-  else if (cd8 && per) launch_update_one<true, true, true, RT>(B, krk, refresh_planes, neg, st);
-  else if (cd8) launch_update_one<true, true, false, RT>(B, krk, refresh_planes, neg, st);
-  else if (per) launch_update_one<true, false, true, RT>(B, krk, refresh_planes, neg, st);
-  else launch_update_one<true, false, false, RT>(B, krk, refresh_planes, neg, st);
-  return hipGetLastError();
+  if (B.du2) return visc_div_update_of<RT, true>(B, krk, refresh_planes, neg, st);
+  return visc_div_update_of<RT, false>(B, krk, refresh_planes, neg, st);
 }
 
 template <typename RT>

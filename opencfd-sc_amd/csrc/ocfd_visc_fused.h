@@ -73,7 +73,7 @@ __host__ __device__ inline int fused_batch_kseg(int nz, int kseg) {
   return k < nz ? k : nz;
 }
 
-template <typename RT>
+template <typename RT, bool TRI>
 __device__ __forceinline__ void visc_fused_tile(const Block &B, const int krk, const int refresh, const int kseg,
                                                 int *neg, int tile) {
   const Geom &g = B.g;
@@ -183,7 +183,7 @@ __device__ __forceinline__ void visc_fused_tile(const Block &B, const int krk, c
   // that uses them ----
   const RT *const dus = reinterpret_cast<const RT *>(B.du);
   struct CellVals {
-    RT du[5];
+    RT du[TRI ? 15 : 5];  // TRI: the three sweeps' parts (tri_du)
     double f[5], fn[5];
   };
   auto fetch_cell = [&](int k) {
@@ -192,6 +192,10 @@ __device__ __forceinline__ void visc_fused_tile(const Block &B, const int krk, c
 #pragma unroll
     for (int m = 0; m < 5; m++) {
       c.du[m] = __builtin_nontemporal_load(&dus[tt + m * ni]);
+      if constexpr (TRI) {
+        c.du[5 + m] = reinterpret_cast<const RT *>(B.du2)[tt + m * ni];
+        c.du[10 + m] = reinterpret_cast<const RT *>(B.du3)[tt + m * ni];
+      }
       c.f[m] = __builtin_nontemporal_load(&B.f[tt + m * ni]);
       c.fn[m] = krk != 1 ? __builtin_nontemporal_load(&B.fn[tt + m * ni]) : 0.0;
     }
@@ -295,7 +299,7 @@ __device__ __forceinline__ void visc_fused_tile(const Block &B, const int krk, c
       double fq[5];
 #pragma unroll
       for (int m = 0; m < 5; m++) {
-        double dum = double(cv.du[m]);
+        double dum = double(TRI ? tri_du(cv.du[m], cv.du[TRI ? 5 + m : 0], cv.du[TRI ? 10 + m : 0], RT(ajac)) : cv.du[m]);
         if (m > 0) dum = dum + double(vd[m]) * ajac;
         const double f = cv.f[m];
         double r;
@@ -344,10 +348,10 @@ __device__ __forceinline__ void visc_fused_tile(const Block &B, const int krk, c
   }
 }
 
-template <typename RT>
+template <typename RT, bool TRI>
 __global__ __launch_bounds__(NT) void k_visc_fused(const Block B, const int krk, const int refresh, const int kseg,
                                                    int *neg) {
-  visc_fused_tile<RT>(B, krk, refresh, kseg, neg, xcd_tile(blockIdx.x, gridDim.x));
+  visc_fused_tile<RT, TRI>(B, krk, refresh, kseg, neg, xcd_tile(blockIdx.x, gridDim.x));
 }
 
 // Batches of periodic boxes (ocfd_batch): the tiles of the launch's boxes in
@@ -360,7 +364,7 @@ __global__ __launch_bounds__(NT) void k_visc_fused_batch(const BoxSet S, const i
   const int j = S.entry(t);
   const int box = S.ids[j];
   const Block B = S.blk[box];  // copied before any store, so its fields stay in scalar registers
-  visc_fused_tile<RT>(B, krk, 1, fused_batch_kseg(B.g.nz, B.kseg), neg + NEG_STRIDE * box, t - S.off[j]);
+  visc_fused_tile<RT, false>(B, krk, 1, fused_batch_kseg(B.g.nz, B.kseg), neg + NEG_STRIDE * box, t - S.off[j]);
 }
 
 template <typename RT>
@@ -369,15 +373,20 @@ hipError_t visc_fused_batch_as(const BoxSet &S, int krk, int *neg, int ntiles, h
   return hipGetLastError();
 }
 
+template <typename RT, bool TRI>
+void visc_fused_one(const Block &B, int krk, int refresh, int *neg, hipStream_t st) {
+  static int cache[64] = {};
+  const int kseg = fused_kseg(B.g, resident_groups(k_visc_fused<RT, TRI>, cache));
+  hipLaunchKernelGGL((k_visc_fused<RT, TRI>), dim3(fused_blocks(B.g, kseg)), dim3(NT), 0, st, B, krk, refresh, kseg, neg);
+}
 template <typename RT>
 hipError_t visc_fused_as(const Block &B, int krk, int refresh, int *neg, hipStream_t st) {
   const Geom &g = B.g;
   if (g.nx % FTX != 0 || g.ny % FTY != 0 || !all_periodic(B) || B.S.scheme_vis == SCH_CD8 || !B.u2.p ||
       !B.v2.p || !B.w2.p)
     return hipErrorInvalidValue;
-  static int cache[64] = {};
-  const int kseg = fused_kseg(g, resident_groups(k_visc_fused<RT>, cache));
-  hipLaunchKernelGGL(k_visc_fused<RT>, dim3(fused_blocks(g, kseg)), dim3(NT), 0, st, B, krk, refresh, kseg, neg);
+  if (B.du2) visc_fused_one<RT, true>(B, krk, refresh, neg, st);
+  else visc_fused_one<RT, false>(B, krk, refresh, neg, st);
   return hipGetLastError();
 }
 
