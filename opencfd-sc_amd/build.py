@@ -25,9 +25,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 ARCH = "gfx950"
 
 SOURCES = ["ocfd_inviscid.hip", "ocfd_inviscid_mixed.hip", "ocfd_inviscid_xyz.hip", "ocfd_inviscid_xyz_mixed.hip",
-           "ocfd_hybrid.hip", "ocfd_viscous.hip",
-           "ocfd_viscous_mixed.hip", "ocfd_misc.hip", "ocfd_batchq.hip", "ocfd_batchq_mixed.hip",
-           "ocfd_api.hip"]
+           "ocfd_inviscid_xy.hip", "ocfd_hybrid.hip", "ocfd_viscous.hip", "ocfd_viscous_mixed.hip", "ocfd_misc.hip",
+           "ocfd_batchq.hip", "ocfd_batchq_mixed.hip", "ocfd_api.hip"]
 
 FLAGS = [
     "--offload-arch=%s" % ARCH, "-O3", "-std=c++17", "-fPIC", "-ffp-contract=off",

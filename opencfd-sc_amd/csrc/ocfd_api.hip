@@ -425,7 +425,9 @@ int inviscid(ocfd_handle *h, bool ch, bool xyz = false) {
   static const char *nm[2][3] = {{"inviscid_x", "inviscid_y", "inviscid_z"},
                                  {"inviscid_char_x", "inviscid_char_y", "inviscid_char_z"}};
   const int modes[3] = {INV_ASSIGN, INV_ACCUM, INV_FINAL};
-  for (int a = 0; a < 3; a++)
+  const bool xy = inviscid_xy_wins(B);
+  if (xy && launch(h, "inviscid_char_xy", [&] { return launch_inviscid_xy(B, h->st); })) return -1;
+  for (int a = xy ? 2 : 0; a < 3; a++)
     if (launch(h, nm[ch][a], [&] { return launch_inviscid(B, a, modes[a], SweepTile{h->tile[a]}, h->st); }))
       return -1;
   return 0;

@@ -162,7 +162,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, weno_lds_t<CHAR,
   const int count = B.hcount[AXIS];
   const int ngroup = (count + NSUB * FB - 1) / (NSUB * FB);  // groups of NSUB batches
   const int *const list = B.hlist[AXIS];
-  double *const out = B.wflux[AXIS];
+  RR *const out = reinterpret_cast<RR *>(B.wflux[AXIS]);
   const bool sw = S.flux_split == 1;
   const bool unif = MET != 0 || B.M.uniform != 0;
   // groups in one contiguous range per XCD (workgroup b runs on XCD
@@ -259,10 +259,10 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, weno_lds_t<CHAR,
       RR x[8];
 #pragma unroll
       for (int k = 0; k < 8; k++) x[k] = F[(row * 8 + k) * FB];
-      const double hp = recon_p(x);
+      const RR hp = recon_p(x);
 #pragma unroll
       for (int k = 0; k < 8; k++) x[k] = F[((5 + row) * 8 + k) * FB];
-      const double hm = recon_m(x);
+      const RR hm = recon_m(x);
       if (f < count) {
         out[(int64_t)f * NH + row] = hp;
         out[(int64_t)f * NH + 5 + row] = hm;
@@ -384,7 +384,7 @@ __device__ __forceinline__ void weno_faces_axis(const Block &B, weno_lds_t<CHAR,
 #pragma unroll
       for (int q = 0; q < 5; q++) h0[q] = sG[q * FB + lane];
       const double hh = madd(sb5[4], h0[4], madd(sb5[3], h0[3], madd(sb5[2], h0[2], madd(sb5[1], h0[1], sb5[0] * h0[0]))));
-      if (f < count) out[(int64_t)f * NH + row] = hh;
+      if (f < count) out[(int64_t)f * NH + row] = RR(hh);
     }
   }
 }

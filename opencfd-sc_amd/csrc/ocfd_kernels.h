@@ -69,7 +69,7 @@ struct Block {
   int *hlist[3], *hcount;
   unsigned long long *hbits[3];
   int *hgbase[3];
-  double *wflux[3];
+  double *wflux[3];  // held in the sweeps' real type
   int prec;  // OCFD_PREC_FP64_CODE / OCFD_PREC_MIXED_CODE (host-side dispatch)
   int kseg;  // boxes of a batch: planes per workgroup of the k-marching kernels
   // Whole-step launches only (NULL otherwise): set by the repair of the first
@@ -281,6 +281,10 @@ struct BLArgs {
 
 // ---- launchers (return hipError_t of the launch) ----
 hipError_t launch_inviscid(const Block &B, int axis, int mode, SweepTile tile, hipStream_t st);
+// the x and y sweeps of a hybrid block in one march (INV_ASSIGN into du), and
+// whether it is faster than the two sweeps
+bool inviscid_xy_wins(const Block &B);
+hipError_t launch_inviscid_xy(const Block &B, hipStream_t st);
 // the three sweeps in one launch, into du, du2 and du3 (no mass force);
 // their join in du
 hipError_t launch_inviscid_xyz(const Block &B, hipStream_t st);
@@ -382,6 +386,21 @@ hipError_t launch_normalise_metrics(const Block &B, double *met[M_N], hipStream_
 
 // threads per workgroup of the element-wise, viscous and stage kernels
 constexpr int NT = 256;
+
+// workgroups of `kernel` (static LDS) the device holds at once;
+// `cache` keeps the value per device for one kernel
+template <typename K>
+int resident_groups(K kernel, int (&cache)[64], int threads = NT) {
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
+  if (cache[dev] == 0) {
+    int cus = 0, per = 0;
+    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess || per < 1) per = 1;
+    cache[dev] = cus * per;
+  }
+  return cache[dev];
+}
 
 // interior (i, j, k), 1-based, of cell t of the nx * ny * nz block (i fastest)
 __device__ inline void cell_of(const Geom &g, int64_t t, int &i, int &j, int &k) {

@@ -130,9 +130,9 @@ __device__ __forceinline__ void march_line(const Block &B, const int i, const in
       if (HYB && ((bits >> bit) & 1ull)) {
         // a listed WENO face (k_weno_faces) replaces the linear one
         const int lslot = B.hgbase[AXIS][fid >> 6] + __popcll(bits & ((1ull << bit) - 1ull));
-        const double *wf = B.wflux[AXIS] + (int64_t)lslot * NH;
+        const R *wf = reinterpret_cast<const R *>(B.wflux[AXIS]) + (int64_t)lslot * NH;
 #pragma unroll
-        for (int q = 0; q < NH; q++) hv[q] = R(wf[q]);
+        for (int q = 0; q < NH; q++) hv[q] = wf[q];
       }
       // ---- cell f: flux difference into du ----
       if (pi >= 8) {

@@ -170,9 +170,9 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
       }
       sS[lidx<AXIS, NF, TW>(0, f, wl)] = slot;
       if (!ALIAS && slot >= 0) {
-        const double *wf = B.wflux[AXIS] + (int64_t)slot * NH;
+        const R *wf = reinterpret_cast<const R *>(B.wflux[AXIS]) + (int64_t)slot * NH;
 #pragma unroll
-        for (int m = 0; m < NH; m++) sH[lidx<AXIS, NF, TW>(m, f, wl)] = R(wf[m]);
+        for (int m = 0; m < NH; m++) sH[lidx<AXIS, NF, TW>(m, f, wl)] = wf[m];
       }
     }
   }
@@ -489,8 +489,8 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
       R v[NV];
       if constexpr (!CHAR) {
         if (HYB && slot_of(f, wl) >= 0) {
-          const double *wf = B.wflux[AXIS] + (int64_t)slot_of(f, wl) * NH;
-          v[0] = R(wf[m]);
+          const R *wf = reinterpret_cast<const R *>(B.wflux[AXIS]) + (int64_t)slot_of(f, wl) * NH;
+          v[0] = wf[m];
           v[1] = R(wf[5 + m]);
         } else {
           face_nc(m, f, wl, s, HYB ? 1 : 0, v[0], v[1]);
@@ -505,7 +505,7 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
       } else if (SPLIT_TAIL && r == NI2 - 1) {
         // hybrid, characteristic, past the whole rounds: component m
         if ((closure_lo && s == 0) || (closure_hi && s == n)) v[0] = closure_comp(f, wl, s, m);
-        else if (slot_of(f, wl) >= 0) v[0] = R(B.wflux[AXIS][(int64_t)slot_of(f, wl) * NH + m]);
+        else if (slot_of(f, wl) >= 0) v[0] = reinterpret_cast<const R *>(B.wflux[AXIS])[(int64_t)slot_of(f, wl) * NH + m];
         else v[0] = linear_comp(f, wl, s, m);
       } else {
         // hybrid, characteristic: the closure, listed and linear faces
@@ -513,9 +513,9 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
 #pragma unroll
           for (int q = 0; q < 5; q++) v[q] = closure_comp(f, wl, s, q);
         } else if (slot_of(f, wl) >= 0) {
-          const double *wf = B.wflux[AXIS] + (int64_t)slot_of(f, wl) * NH;
+          const R *wf = reinterpret_cast<const R *>(B.wflux[AXIS]) + (int64_t)slot_of(f, wl) * NH;
 #pragma unroll
-          for (int q = 0; q < 5; q++) v[q] = R(wf[q]);
+          for (int q = 0; q < 5; q++) v[q] = wf[q];
         } else {
 #pragma unroll
           for (int q = 0; q < 5; q++) v[q] = linear_comp(f, wl, s, q);

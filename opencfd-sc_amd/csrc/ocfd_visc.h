@@ -572,21 +572,6 @@ __global__ __launch_bounds__(NT) void k_visc_div_update_batch(const BoxSet S, co
 // ---------------------------------------------------------------------------
 inline unsigned nblocks(int64_t n) { return (unsigned)((n + NT - 1) / NT); }
 
-// workgroups of `kernel` (NT threads, static LDS) the device holds at once;
-// `cache` keeps the value per device for one kernel
-template <typename K>
-int resident_groups(K kernel, int (&cache)[64]) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (cache[dev] == 0) {
-    int cus = 0, per = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, NT, 0) != hipSuccess || per < 1) per = 1;
-    cache[dev] = cus * per;
-  }
-  return cache[dev];
-}
-
 // Planes per workgroup of a k-marching kernel: its time is close to the
 // number of rounds of resident workgroups times the planes of a segment plus
 // its prologue (the plane queue and the first tile, about 2.5 planes: 6.3 +
