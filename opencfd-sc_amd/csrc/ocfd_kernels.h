@@ -404,10 +404,17 @@ int resident_groups(K kernel, int (&cache)[64], int threads = NT) {
 
 // interior (i, j, k), 1-based, of cell t of the nx * ny * nz block (i fastest)
 __device__ inline void cell_of(const Geom &g, int64_t t, int &i, int &j, int &k) {
-  i = (int)(t % g.nx) + 1;
-  int64_t r = t / g.nx;
-  j = (int)(r % g.ny) + 1;
-  k = (int)(r / g.ny) + 1;
+  if (g.ni <= INT32_MAX) {  // (a 64-bit division takes some 100 instructions)
+    const unsigned q = (unsigned)t / (unsigned)g.nx, r = q / (unsigned)g.ny;
+    i = (int)((unsigned)t - q * (unsigned)g.nx) + 1;
+    j = (int)(q - r * (unsigned)g.ny) + 1;
+    k = (int)r + 1;
+  } else {
+    i = (int)(t % g.nx) + 1;
+    int64_t r = t / g.nx;
+    j = (int)(r % g.ny) + 1;
+    k = (int)(r / g.ny) + 1;
+  }
 }
 
 }  // namespace ocfd

@@ -43,7 +43,7 @@ template <typename E>
 __global__ __launch_bounds__(NT) void k_sensor1(const Block B, const double p00) {
   const Geom &g = B.g;
   const E *const pd = B.d.as<E>(), *const pT = B.T.as<E>();
-  const int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
+  const int64_t t = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;
   if (t >= g.ni) return;
   int i, j, k;
   cell_of(g, t, i, j, k);
@@ -402,8 +402,7 @@ __global__ __launch_bounds__(NT) void k_bl_sides(const Block B, const BLArgs a) 
 }
 
 // f recomputed from the primitives on the six block faces (OCFD_BC.f90:26-95)
-__global__ __launch_bounds__(NT) void k_bc_planes(const Block B) {
-  if (halted(B)) return;  // a whole-step run stopped at too many T <= 0 cells
+__device__ __forceinline__ void bc_planes(const Block &B) {
   const Geom &g = B.g;
   const int64_t ax = (int64_t)g.ny * g.nz, ay = (int64_t)g.nx * g.nz, az = (int64_t)g.nx * g.ny;
   int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
@@ -431,8 +430,7 @@ __global__ __launch_bounds__(NT) void k_bc_planes(const Block B) {
 }
 
 // Flow_Ghost_Extent_2nd (OCFD_GhostCell.f90:164-286)
-__global__ __launch_bounds__(NT) void k_ghost(const Block B, const int side) {
-  if (halted(B)) return;  // a whole-step run stopped at too many T <= 0 cells
+__device__ __forceinline__ void ghost_side(const Block &B, const int side) {
   const Geom &g = B.g;
   const int axis = side / 2, hi = side % 2;
   const int a1 = axis == 0 ? 1 : 0, a2 = axis == 2 ? 1 : 2;  // the two other axes
@@ -468,8 +466,7 @@ __global__ __launch_bounds__(NT) void k_ghost(const Block B, const int side) {
 // boundary layer; mirror about j = 1 with the 0.5 / 2.0 limiter,
 // Flow_Ghost_flatplate :110-136) or swept-corner symmetry plane k- (w
 // changes sign, Flow_Ghost_Sweptcorner :56-76)
-__global__ __launch_bounds__(NT) void k_ghost_user(const Block B, const int ibc) {
-  if (halted(B)) return;  // a whole-step run stopped at too many T <= 0 cells
+__device__ __forceinline__ void ghost_user(const Block &B, const int ibc) {
   const Geom &g = B.g;
   const int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
   if (ibc == 2) {
@@ -506,6 +503,22 @@ __global__ __launch_bounds__(NT) void k_ghost_user(const Block B, const int ibc)
   }
 }
 
+// What follows the boundary conditions, one part per blockIdx.y: f on the block
+// faces and the ghost layers of each side.  A part reads interior points and
+// block faces of the primitives and writes f or its own ghost layer, so the
+// parts are independent.  (One launch each: boundary layer of 240 x 100 x 48,
+// 41 us a stage with the conditions, 35 in one.)
+struct AfterBc {
+  int n, part[8];  // 0-5 ghost side, 6 and 7 user ghost layers (j-, k-), 8 block faces
+};
+__global__ __launch_bounds__(NT) void k_after_bc(const Block B, const AfterBc A) {
+  if (halted(B)) return;  // a whole-step run stopped at too many T <= 0 cells
+  const int q = A.part[blockIdx.y];
+  if (q < 6) ghost_side(B, q);
+  else if (q < 8) ghost_user(B, q - 4);
+  else bc_planes(B);
+}
+
 // ---------------------------------------------------------------------------
 // filters: out-of-place along one axis; cells outside the filtered index box
 // are copied unchanged
@@ -515,9 +528,11 @@ struct FilterArgs {
   double s0, rth;
   int lo[3], hi[3];
 };
+// Fo9p: one component per blockIdx.y, tiles of a plane range per XCD (240 x 100
+// x 48, three axes: 54 us a launch with the five components in a loop, 44 now).
 __global__ __launch_bounds__(NT) void k_filter(const Block B, const FilterArgs A, double *fout) {
   const Geom &g = B.g;
-  const int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
+  const int64_t t = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;
   if (t >= g.ni) return;
   int idx[3];
   cell_of(g, t, idx[0], idx[1], idx[2]);
@@ -528,7 +543,7 @@ __global__ __launch_bounds__(NT) void k_filter(const Block B, const FilterArgs A
   const bool in = !halted(B) && idx[0] >= A.lo[0] && idx[0] <= A.hi[0] && idx[1] >= A.lo[1] &&
                   idx[1] <= A.hi[1] && idx[2] >= A.lo[2] && idx[2] <= A.hi[2];
   auto wrap = [&](int q) { return q < 1 ? q + n : (q > n ? q - n : q); };
-  for (int m = 0; m < 5; m++) {
+  for (int m = blockIdx.y; m < 5; m += gridDim.y) {
     const double *f0 = B.f + (int64_t)m * ni;
     double r = f0[t];
     if (in) {
@@ -993,20 +1008,22 @@ hipError_t launch_bc(const Block &B, int ibc, double tw, const BLArgs *bl, const
     if (ibc == 3 && (bl->z1 == 1 || bl->z2 == 1))
       hipLaunchKernelGGL(k_bl_sides, dim3(nb((int64_t)g.nx * g.ny)), dim3(NT), 0, st, B, *bl);
   }
-  const int64_t np = 2 * ((int64_t)g.ny * g.nz + (int64_t)g.nx * g.nz + (int64_t)g.nx * g.ny);
-  if (planes) hipLaunchKernelGGL(k_bc_planes, dim3(nb(np)), dim3(NT), 0, st, B);
-  for (int side = 0; side < 6; side++) {
-    if (ghost[side] != 1 && ghost[side] != 2) continue;
-    const int axis = side / 2;
-    const int64_t cnt = (int64_t)LAP * (axis == 0 ? (int64_t)g.ny * g.nz : (axis == 1 ? (int64_t)g.nx * g.nz : (int64_t)g.nx * g.ny));
-    hipLaunchKernelGGL(k_ghost, dim3(nb(cnt)), dim3(NT), 0, st, B, side);
-  }
+  AfterBc A;
+  A.n = 0;
+  int64_t most = 0;
+  auto part = [&](int q, int64_t cnt) {
+    A.part[A.n++] = q;
+    if (cnt > most) most = cnt;
+  };
+  const int64_t ax = (int64_t)g.ny * g.nz, ay = (int64_t)g.nx * g.nz, az = (int64_t)g.nx * g.ny;
+  if (planes) part(8, 2 * (ax + ay + az));
+  for (int side = 0; side < 6; side++)
+    if (ghost[side] == 1 || ghost[side] == 2) part(side, LAP * (side < 2 ? ax : (side < 4 ? ay : az)));
   // user ghost layers (Ghost_Cell = -1): flat plate j- / swept corner k-
   const int ibc_any = ibc < 0 ? -ibc : ibc;
-  if (ibc_any == 2 && ghost[2] == -1)
-    hipLaunchKernelGGL(k_ghost_user, dim3(nb((int64_t)LAP * g.nx * g.nz)), dim3(NT), 0, st, B, 2);
-  if (ibc_any == 3 && ghost[4] == -1)
-    hipLaunchKernelGGL(k_ghost_user, dim3(nb((int64_t)LAP * g.nx * g.ny)), dim3(NT), 0, st, B, 3);
+  if (ibc_any == 2 && ghost[2] == -1) part(6, LAP * ay);
+  if (ibc_any == 3 && ghost[4] == -1) part(7, LAP * az);
+  if (A.n) hipLaunchKernelGGL(k_after_bc, dim3(nb(most), (unsigned)A.n), dim3(NT), 0, st, B, A);
   return hipGetLastError();
 }
 
@@ -1025,7 +1042,7 @@ hipError_t launch_filter(const Block &B, int axis, int scheme, double s0, double
     if (A.lo[axis] < lo_min) A.lo[axis] = lo_min;
     if (A.hi[axis] > n - hi_off) A.hi[axis] = n - hi_off;
   }
-  hipLaunchKernelGGL(k_filter, dim3(nb(B.g.ni)), dim3(NT), 0, st, B, A, fout);
+  hipLaunchKernelGGL(k_filter, dim3(nb(B.g.ni), scheme == 1 ? 5 : 1), dim3(NT), 0, st, B, A, fout);
   return hipGetLastError();
 }
 
