@@ -43,7 +43,7 @@ template <typename E>
 __global__ __launch_bounds__(NT) void k_sensor1(const Block B, const double p00) {
   const Geom &g = B.g;
   const E *const pd = B.d.as<E>(), *const pT = B.T.as<E>();
-  const int64_t t = (int64_t)xcd_tile(blockIdx.x, gridDim.x) * NT + threadIdx.x;
+  const int64_t t = (int64_t)blockIdx.x * NT + threadIdx.x;
   if (t >= g.ni) return;
   int i, j, k;
   cell_of(g, t, i, j, k);
