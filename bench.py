@@ -240,8 +240,11 @@ KERNEL_SYMBOL = {"stage_update": "k_visc_div_update", "stage_update_fused": "k_v
                  "visc_flux": "k_visc_flux", "halo_fill": "k_halo",
                  "inviscid_x": "k_inviscid<0", "inviscid_y": "k_inviscid<1", "inviscid_z": "k_inviscid<2",
                  "inviscid_char_x": "k_inviscid<0", "inviscid_char_y": "k_inviscid<1",
-                 "inviscid_char_z": "k_inviscid<2", "weno_faces": "k_weno_faces", "sensor": "k_sensor1",
+                 "inviscid_char_z": "k_inviscid<2", "inviscid_char_xy": "k_inviscid_xy<",
+                 "inviscid_xyz": "k_inviscid_xyz<", "weno_faces": "k_weno_faces", "sensor": "k_sensor1",
                  "hyb_list": "k_hyb_list"}
+# axes that one launch of a sweep kernel covers, where not one
+LAUNCH_AXES = {"inviscid_char_xy": 2, "inviscid_xyz": 3, "weno_faces": 3}
 
 
 def profile_traffic(workload: str, precision: str, name: str):
@@ -319,13 +322,14 @@ def kernel_roofline(name, ms, cnt, cfg, variant, mix, prec, workload):
     rb = 4 if prec == PREC_MIXED else 8
     peak_f = perfmodel.PEAK_FP64_TFLOPS if prec == PREC_FP64 else perfmodel.PEAK_FP32_TFLOPS
     if name.startswith("inviscid") or name == "weno_faces":
+        axes = LAUNCH_AXES.get(name, 1)
         if name == "weno_faces":
-            flops = perfmodel.weno_faces_axis_flops(variant, n, mix)
+            flops = axes * perfmodel.weno_faces_axis_flops(variant, n, mix)
         else:
-            flops = perfmodel.inviscid_axis_flops(variant, n, mix)
-            if name == "inviscid_char_x" or name == "inviscid_char_y" or name == "inviscid_char_z":
+            flops = axes * perfmodel.inviscid_axis_flops(variant, n, mix)
+            if name.startswith("inviscid_char_"):
                 # the sweeps compute the linear faces; the listed WENO faces are k_weno_faces'
-                flops -= perfmodel.weno_faces_axis_flops(variant, n, mix)
+                flops -= axes * perfmodel.weno_faces_axis_flops(variant, n, mix)
         ach = flops / avg_s / 1e12
         roof = {"bound": "valu", "achieved": round(ach, 3), "peak": peak_f, "unit": "TFLOP/s",
                 "frac": round(ach / peak_f, 4), "kernel": name, "algorithmic_per_launch": flops,
