@@ -3,6 +3,8 @@
 // Same arithmetic as the two sweeps one after the other (ocfd_sweep.h,
 // ocfd_march.h; du_inviscous_Character, OCFD_inviscous_character.f90:3-159):
 // du = x part + y part, for the z sweep to add to.
+#include <algorithm>
+
 #include "ocfd_kernels.h"
 
 namespace ocfd {
@@ -148,7 +150,7 @@ void k_inviscid_xy(const Block B, const int sl) {
     const int bit = (int)(fid & 63);
     const bool y = ((e.bits >> bit) & 1ull) != 0;
     const unsigned slot = (unsigned)(e.base + __popcll(e.bits & ((1ull << bit) - 1ull)));
-    at = y ? slot * 5u : 0u;
+    at = y ? slot * 5u : 0u;  // (inviscid_xy_wins bounds it)
     return y;
   };
   const R *const wfx = reinterpret_cast<const R *>(B.wflux[0]), *const wfy = reinterpret_cast<const R *>(B.wflux[1]);
@@ -337,9 +339,13 @@ hipError_t inviscid_xy_as(const Block &B, hipStream_t st) {
 // 128^3 (1.5) 66 and 48, 200 x 180 x 150 (1.75) 176 and 134, 100 x 140 x 120
 // (2.5) 57 and 60.  Steger-Warming in FP64 needs more registers than there
 // are: 256^3 (1.3) 840 and 777, 160^3 219 and 240.
+// It addresses the five fluxes of a listed face with 32 bits, so blocks with
+// more faces per axis than that reaches (ocfd_create accepts up to 2^30) take
+// the two sweeps.
 bool inviscid_xy_wins(const Block &B) {
   if (B.S.scheme_invis != SCH_HYBRID || !B.S.is_char || B.S.iperiodic[0] != 1 || B.S.iperiodic[1] != 1 || !B.M.uniform)
     return false;
+  if (5 * std::max(TileIndex<0>::nfaces(B.g), TileIndex<1>::nfaces(B.g)) > (int64_t)UINT32_MAX) return false;
   const bool f32 = B.prec == OCFD_PREC_MIXED_CODE, sw = B.S.flux_split == 1;
   int64_t work;
   if (f32) sw ? xy_segment<float, true>(B.g, work) : xy_segment<float, false>(B.g, work);
