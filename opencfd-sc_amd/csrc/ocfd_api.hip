@@ -1857,13 +1857,16 @@ int ocfd_batch_box(ocfd_batch *b, int32_t i, ocfd_handle **h) {
 
 int ocfd_batch_step(ocfd_batch *b, int32_t nsteps) {
   const int nbox = (int)b->box.size();
+  // (a box that stepped alone; the tables' update waits for its stream)
+  HIPCHK(hipSetDevice(b->device));
+  for (ocfd_handle *h : b->box)
+    if (settle_du(h)) return -1;
   if (batch_sync_tables(b)) return -1;
   hipLaunchKernelGGL(k_zero_int, dim3((unsigned)((NEG_STRIDE * nbox + 127) / 128)), dim3(128), 0, b->st, b->neg,
                      NEG_STRIDE * nbox);
   std::vector<int> istep0(nbox);
   std::vector<double> tt0(nbox);
   for (int i = 0; i < nbox; i++) {
-    b->box[i]->du_parts = false;  // the batch's sweeps write du itself
     istep0[i] = b->box[i]->istep;
     tt0[i] = b->box[i]->tt;
   }
@@ -1968,6 +1971,9 @@ int ocfd_batch_info(ocfd_batch *b, int32_t *ngroups, int32_t *shapes, int64_t *c
 
 int ocfd_batch_autotune(ocfd_batch *b, int32_t reps) {
   if (reps < 1) reps = 5;
+  HIPCHK(hipSetDevice(b->device));
+  for (ocfd_handle *h : b->box)
+    if (settle_du(h)) return -1;
   if (batch_sync_tables(b)) return -1;
   if (batch_halo(b)) return -1;
   hipEvent_t e0, e1;
