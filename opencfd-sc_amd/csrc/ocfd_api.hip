@@ -74,8 +74,10 @@ struct ocfd_handle {
   // and the repair copies none (mixed 256^3: repair 61 -> 4 us per stage)
   bool halo_both = false;
   // small blocks: the y and z parts of du of whole steps, whose three sweeps
-  // are one launch (k_inviscid_xyz); NULL where the sweeps run one by one
-  double *du_yz = nullptr;
+  // are one launch (k_inviscid_xyz), in the sweeps' real type; allocated by the
+  // first whole step (ensure_parts), NULL where the sweeps run one by one
+  char *du_yz = nullptr;
+  bool parts_tried = false;
   bool du_parts = false;  // du holds the x part alone (settle_du joins them)
   // per-routine calls merged into the whole-step stage kernels
   // (ocfd_set_stage_fusion); pend holds what the stage so far left to do
@@ -86,6 +88,7 @@ struct ocfd_handle {
   std::map<std::string, std::pair<double, long long>> acc;
   size_t halo_bytes() const { return (size_t)B.g.nh * sizeof(double); }
   size_t f_bytes() const { return (size_t)5 * B.g.ni * sizeof(double); }
+  size_t part_bytes() const { return B.prec == OCFD_PREC_MIXED_CODE ? f_bytes() / 2 : f_bytes(); }
 };
 
 namespace {
@@ -398,9 +401,27 @@ int upload_prims(ocfd_handle *h, const double *const src[5], bool make_f) {
 
 // a block whose right-hand side is in the three sweeps' parts
 Block with_parts(const ocfd_handle *h, Block B) {
-  B.du2 = h->du_yz;
-  B.du3 = h->du_yz + 5 * B.g.ni;
+  B.du2 = reinterpret_cast<double *>(h->du_yz);
+  B.du3 = reinterpret_cast<double *>(h->du_yz + h->part_bytes());
   return B;
+}
+// Room for the parts, on the first whole step: the boxes of a batch, whose
+// sweeps run one by one, and blocks driven by the routines never need it, and
+// every block's own arrays come first.  Without room the sweeps run one by one.
+// (The mass force is added by the z sweep.)
+int ensure_parts(ocfd_handle *h) {
+  if (h->parts_tried) return 0;
+  h->parts_tried = true;
+  if (h->B.g.ni > XYZ_MAX_CELLS || h->cfg.if_mass_force == 1) return 0;
+  int cur = 0;
+  HIPCHK(hipGetDevice(&cur));
+  if (cur != h->device) HIPCHK(hipSetDevice(h->device));
+  if (hipMalloc((void **)&h->du_yz, 2 * h->part_bytes()) != hipSuccess) {
+    h->du_yz = nullptr;
+    (void)hipGetLastError();
+  }
+  if (cur != h->device) HIPCHK(hipSetDevice(cur));
+  return 0;
 }
 // du as the z sweep leaves it, for its readers outside whole steps
 int settle_du(ocfd_handle *h) {
@@ -569,12 +590,6 @@ int ocfd_create(const ocfd_config *cfg, int device, ocfd_handle **out) {
   B.halt = nullptr;
   B.du2 = B.du3 = nullptr;
   rc |= alloc(&B.f, fb) | alloc(&B.fn, fb) | alloc(&B.du, fb);
-  // without room for it the sweeps run one by one
-  // (the mass force is added by the z sweep)
-  if (B.g.ni <= XYZ_MAX_CELLS && cfg->if_mass_force != 1 && hipMalloc((void **)&h->du_yz, 2 * fb) != hipSuccess) {
-    h->du_yz = nullptr;
-    (void)hipGetLastError();
-  }
   if (cfg->scheme_invis == SCH_HYBRID) rc |= alloc(&B.rhyb, hb);
   if (cfg->if_viscous == 1) rc |= alloc(&B.ev, 12 * (size_t)B.g.ni * sizeof(double));
   if (cfg->nfiltering > 0) rc |= alloc(&h->fbuf, fb);
@@ -655,9 +670,10 @@ int ocfd_destroy(ocfd_handle *h) {
   Block &B = h->B;
   for (const PrimField *p : {&B.d, &B.u, &B.v, &B.w, &B.T, &B.T2, &B.u2, &B.v2, &B.w2})
     if (p->p) (void)hipFree(p->p);
-  double *ps[] = {B.f, B.fn, B.du, h->du_yz, B.rhyb, B.ev, h->fbuf, h->work, h->wout};
+  double *ps[] = {B.f, B.fn, B.du, B.rhyb, B.ev, h->fbuf, h->work, h->wout};
   for (double *p : ps)
     if (p) (void)hipFree(p);
+  if (h->du_yz) (void)hipFree(h->du_yz);
   for (int a = 0; a < 3; a++) {
     if (B.hlist[a]) (void)hipFree(B.hlist[a]);
     if (B.hbits[a]) (void)hipFree(B.hbits[a]);
@@ -1210,6 +1226,7 @@ void invalidate_graph(ocfd_handle *h) {
 int ocfd_step(ocfd_handle *h, int32_t nsteps) {
   const ocfd_config &c = h->cfg;
   h->pend = 0;
+  if (ensure_parts(h)) return -1;
   hipLaunchKernelGGL(k_zero_int, dim3(1), dim3(128), 0, h->st, h->neg, NEG_STRIDE);
   // filtering decides per step on the host; per-kernel timing needs eager launches
   const bool graph = h->use_graph && !h->prof && c.nfiltering == 0;
