@@ -240,17 +240,22 @@ int ocfd_advance_clock(ocfd_handle *h);
 int ocfd_step(ocfd_handle *h, int32_t nsteps);
 
 /* ---- sweep tiles (no counterpart in the reference) --------------------- */
-/* Tile shape of the inviscid sweep of each axis: 0 = x 64x4, y/z 32x8 points
- * x lines (the default); 1 = x 32x8, y/z 16x16; 2 = x 128x2, y/z 64x4;
- * 3 and 4 (y and z only) march along the axis, one lane per line, over
- * segments of 32 and 64 points, keeping the split fluxes in registers.
- * Shapes 1-4 apply to periodic axes with OCFD_METRIC_UNIFORM whose extents
- * fit them; other axes use 0.  Results are bit-identical for every shape. */
+/* Tile shape of the inviscid sweep of each axis: 0 = left to the library (the
+ * default: x 64x4, y/z 32x8 points x lines, or the tuner's); 1 = x 32x8, y/z
+ * 16x16; 2 = x 128x2, y/z 64x4; 3 and 4 (y and z only) march along the axis,
+ * one lane per line, over segments of 32 and 64 points, keeping the split
+ * fluxes in registers.  Shapes 1-4 apply to periodic axes with
+ * OCFD_METRIC_UNIFORM whose extents fit them; other axes use 0.  With 0 the
+ * library may run sweeps together in one launch: all three in the whole steps
+ * of small blocks (the three shapes 0), x and y of periodic hybrid
+ * characteristic blocks that fill the chip (x and y 0).  Results are
+ * bit-identical for every shape. */
 int ocfd_set_sweep_tiles(ocfd_handle *h, const int32_t shape[3]);
 int ocfd_get_sweep_tiles(ocfd_handle *h, int32_t shape[3]);
 /* Autotuner: times `reps` launches of each axis' sweep in every shape it
- * supports on the block's current state and keeps the fastest (shape_out may
- * be NULL).  Overwrites du (a work array): call it between time steps. */
+ * supports on the block's current state, and of the launch of x and y, and
+ * keeps the fastest: shape_out (may be NULL) is 0 for axes that run together.
+ * Overwrites du (a work array): call it between time steps. */
 int ocfd_autotune(ocfd_handle *h, int32_t reps, int32_t shape_out[3]);
 
 /* ---- diagnostics ------------------------------------------------------ */

@@ -38,6 +38,21 @@ struct ProfRec {
   std::string name;
   hipEvent_t a, b;
 };
+
+// Whole steps of blocks up to XYZ_MAX_CELLS run their three sweeps in one launch
+// (k_inviscid_xyz).  A sweep of a small block does not fill the chip and its
+// launch costs as much as its arithmetic; of a larger one the launches are a
+// few percent, and the two more arrays that the stage update reads cost more
+// than they save.  Step times, three launches (tuned tiles) and one, us: WENO5
+// 32^3 127 and 95, 64^3 286 and 255, 80^3 530 and 489; WENO7 characteristic
+// 32^3 163 and 122, 80^3 811 and 754, 120 x 100 x 48 825 and 805; OMP6 80^3 507
+// and 468; hybrid 80^3 563 and 539, mixed precision 390 and 363.  Beyond: WENO7
+// characteristic 96^3 1172 and 1180, 104^3 1565 and 1611; hybrid 96^3 1728 and
+// 1733, 112^3 2077 and 2151; WENO5 characteristic plate 200 x 100 x 40 1608 and
+// 1610.
+// (The mass force is added by the z sweep.)
+constexpr int64_t XYZ_MAX_CELLS = 600000;
+bool xyz_wins(const Block &B) { return B.P.if_mass_force != 1 && B.g.ni <= XYZ_MAX_CELLS; }
 }  // namespace
 
 struct ocfd_handle {
@@ -58,7 +73,14 @@ struct ocfd_handle {
   double tt = 0.0;
   bool prof = false;
   bool use_graph = true;           // replay whole steps from a captured hipGraph
-  int tile[3] = {0, 0, 0};         // sweep tile shape per axis (SweepTile)
+  // sweep tile shape per axis (SweepTile).  Not 0: the axis' sweep runs in a
+  // launch of its own with this shape.  0: left to the library, which may join
+  // sweeps in one launch; where the sweep runs by itself all the same (the
+  // routines of a block whose whole steps join them), in the shape `tuned`
+  int tile[3] = {0, 0, 0};
+  int tuned[3] = {0, 0, 0};
+  bool xy_slower = false;          // the tuner found two sweeps faster than the x-y march
+  int shape(int a) const { return tile[a] ? tile[a] : tuned[a]; }
   BLArgs bl = {};                  // boundary-layer / swept-corner data (ibc 2, 3)
   bool bl_set = false;
   std::vector<void *> bl_mem;      // its device arrays
@@ -78,6 +100,11 @@ struct ocfd_handle {
   // first whole step (ensure_parts), NULL where the sweeps run one by one
   char *du_yz = nullptr;
   bool parts_tried = false;
+  // whole steps take the three sweeps in one launch, once there is room
+  bool joins_xyz() const { return !tile[0] && !tile[1] && !tile[2] && (du_yz || !parts_tried) && xyz_wins(B); }
+  bool joined_xyz() const { return du_yz && joins_xyz(); }
+  // x and y in one march
+  bool joins_xy(const Block &b) const { return !tile[0] && !tile[1] && !xy_slower && inviscid_xy_wins(b); }
   bool du_parts = false;  // du holds the x part alone (settle_du joins them)
   // per-routine calls merged into the whole-step stage kernels
   // (ocfd_set_stage_fusion); pend holds what the stage so far left to do
@@ -286,18 +313,6 @@ __global__ void k_patch(const Geom g, double *r, int ib, int ie, int jb, int je,
   r[q] = r[q] + 100.0;
 }
 
-// Whole steps of blocks up to this size run their three sweeps in one launch
-// (k_inviscid_xyz).  A sweep of a small block does not fill the chip and its
-// launch costs as much as its arithmetic; of a larger one the launches are a
-// few percent, and the two more arrays that the stage update reads cost more
-// than they save.  Step times, three launches and one, us: WENO5 32^3 130 and
-// 95, 64^3 291 and 265, 96^3 780 and 742; WENO7 characteristic 32^3 183 and
-// 122, 80^3 815 and 760, 96^3 1172 and 1180, 104^3 1565 and 1611; hybrid, tuned
-// tiles, 80^3 1078 and 1054, 96^3 1728 and 1733, 112^3 2077 and 2151; in mixed
-// precision 80^3 704 and 675, 104^3 1238 and 1241; WENO5 characteristic plate
-// 120 x 100 x 48 1206 and 1180, 200 x 100 x 40 1608 and 1610.
-constexpr int64_t XYZ_MAX_CELLS = 600000;
-
 int alloc(double **p, size_t bytes) {
   if (hipMalloc((void **)p, bytes) != hipSuccess) {
     *p = nullptr;
@@ -408,11 +423,9 @@ Block with_parts(const ocfd_handle *h, Block B) {
 // Room for the parts, on the first whole step: the boxes of a batch, whose
 // sweeps run one by one, and blocks driven by the routines never need it, and
 // every block's own arrays come first.  Without room the sweeps run one by one.
-// (The mass force is added by the z sweep.)
 int ensure_parts(ocfd_handle *h) {
-  if (h->parts_tried) return 0;
+  if (h->parts_tried || !h->joins_xyz()) return 0;
   h->parts_tried = true;
-  if (h->B.g.ni > XYZ_MAX_CELLS || h->cfg.if_mass_force == 1) return 0;
   int cur = 0;
   HIPCHK(hipGetDevice(&cur));
   if (cur != h->device) HIPCHK(hipSetDevice(h->device));
@@ -446,10 +459,10 @@ int inviscid(ocfd_handle *h, bool ch, bool xyz = false) {
   static const char *nm[2][3] = {{"inviscid_x", "inviscid_y", "inviscid_z"},
                                  {"inviscid_char_x", "inviscid_char_y", "inviscid_char_z"}};
   const int modes[3] = {INV_ASSIGN, INV_ACCUM, INV_FINAL};
-  const bool xy = inviscid_xy_wins(B);
+  const bool xy = h->joins_xy(B);
   if (xy && launch(h, "inviscid_char_xy", [&] { return launch_inviscid_xy(B, h->st); })) return -1;
   for (int a = xy ? 2 : 0; a < 3; a++)
-    if (launch(h, nm[ch][a], [&] { return launch_inviscid(B, a, modes[a], SweepTile{h->tile[a]}, h->st); }))
+    if (launch(h, nm[ch][a], [&] { return launch_inviscid(B, a, modes[a], SweepTile{h->shape(a)}, h->st); }))
       return -1;
   return 0;
 }
@@ -1163,7 +1176,7 @@ int step_body(ocfd_handle *h) {
   for (int krk = 1; krk <= 3; krk++) {
     if (h->halo_both ? exchange_stage(h) : exchange_prims(h)) return -1;
     if (krk == 1 && hyb && sensor(h)) return -1;
-    const bool xyz = h->du_yz != nullptr;
+    const bool xyz = h->joined_xyz();
     if (inviscid(h, ch, xyz)) return -1;
     const int refresh = h->ibc == 0 ? 1 : 0;
     Block B = xyz ? with_parts(h, h->B) : h->B;
@@ -1248,7 +1261,7 @@ int ocfd_step(ocfd_handle *h, int32_t nsteps) {
         if (h->fused) swap_uvw(h);
       }
       if (!rc && hipGraphLaunch(h->gexec[p], h->st) != hipSuccess) rc = fail("hipGraphLaunch failed");
-      h->du_parts = h->du_yz != nullptr;
+      h->du_parts = h->joined_xyz();
     } else {
       rc = step_body(h);
     }
@@ -1286,7 +1299,11 @@ int ocfd_step(ocfd_handle *h, int32_t nsteps) {
 int ocfd_set_sweep_tiles(ocfd_handle *h, const int32_t shape[3]) {
   for (int a = 0; a < 3; a++)
     if (shape[a] < 0 || shape[a] >= NSWEEP_SHAPES) return fail("sweep tile shape must be 0 .. 4");
-  for (int a = 0; a < 3; a++) h->tile[a] = shape[a];
+  for (int a = 0; a < 3; a++) {
+    h->tile[a] = shape[a];
+    h->tuned[a] = 0;
+  }
+  h->xy_slower = false;
   invalidate_graph(h);
   return 0;
 }
@@ -1295,6 +1312,21 @@ int ocfd_get_sweep_tiles(ocfd_handle *h, int32_t shape[3]) {
   for (int a = 0; a < 3; a++) shape[a] = h->tile[a];
   return 0;
 }
+
+}  // extern "C"
+namespace {
+// `reps` launches after one to warm up, ms in all
+template <typename F>
+hipError_t time_launches(ocfd_handle *h, int reps, F &&fn, hipEvent_t e0, hipEvent_t e1, float *ms) {
+  hipError_t e = fn();
+  e = e != hipSuccess ? e : hipEventRecord(e0, h->st);
+  for (int r = 0; r < reps && e == hipSuccess; r++) e = fn();
+  e = e != hipSuccess ? e : hipEventRecord(e1, h->st);
+  e = e != hipSuccess ? e : hipEventSynchronize(e1);
+  return e != hipSuccess ? e : hipEventElapsedTime(ms, e0, e1);
+}
+}  // namespace
+extern "C" {
 
 int ocfd_autotune(ocfd_handle *h, int32_t reps, int32_t shape_out[3]) {
   if (reps < 1) reps = 5;
@@ -1317,6 +1349,7 @@ int ocfd_autotune(ocfd_handle *h, int32_t reps, int32_t shape_out[3]) {
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   rc = 0;
+  float alone = 0.f;  // the x and y sweeps in their best shapes
   for (int a = 0; a < 3 && !rc; a++) {
     // the alternative shapes exist for periodic axes with uniform metrics
     // (the marches for the y and z sweeps of some schemes)
@@ -1325,13 +1358,9 @@ int ocfd_autotune(ocfd_handle *h, int32_t reps, int32_t shape_out[3]) {
     int bests = 0;
     for (int sh = 0; sh < NSWEEP_SHAPES && !rc; sh++) {
       if (!sweep_shape_supported(a, sh, fast, c.scheme_invis, ch)) continue;
-      hipError_t e = launch_inviscid(B, a, modes[a], SweepTile{sh}, h->st);  // warm-up
-      e = e != hipSuccess ? e : hipEventRecord(e0, h->st);
-      for (int r = 0; r < reps && e == hipSuccess; r++) e = launch_inviscid(B, a, modes[a], SweepTile{sh}, h->st);
-      e = e != hipSuccess ? e : hipEventRecord(e1, h->st);
-      e = e != hipSuccess ? e : hipEventSynchronize(e1);
       float ms = 0.f;
-      e = e != hipSuccess ? e : hipEventElapsedTime(&ms, e0, e1);
+      const hipError_t e =
+          time_launches(h, reps, [&] { return launch_inviscid(B, a, modes[a], SweepTile{sh}, h->st); }, e0, e1, &ms);
       if (e != hipSuccess) {
         rc = fail(std::string("autotune: ") + hipGetErrorString(e));
         break;
@@ -1341,11 +1370,25 @@ int ocfd_autotune(ocfd_handle *h, int32_t reps, int32_t shape_out[3]) {
         bests = sh;
       }
     }
-    h->tile[a] = bests;
+    h->tuned[a] = bests;
+    alone += a < 2 ? best : 0.f;
+  }
+  // the two sweeps against the x-y march
+  h->xy_slower = false;
+  if (!rc && inviscid_xy_wins(B)) {
+    float ms = 0.f;
+    const hipError_t e = time_launches(h, reps, [&] { return launch_inviscid_xy(B, h->st); }, e0, e1, &ms);
+    if (e != hipSuccess) rc = fail(std::string("autotune: ") + hipGetErrorString(e));
+    h->xy_slower = alone < ms;
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   if (rc) return -1;
+  // 0 for the axes that whole steps join
+  for (int a = 0; a < 3; a++) h->tile[a] = 0;
+  const bool xyz = h->joins_xyz(), xy = h->joins_xy(B);
+  for (int a = 0; a < 3; a++)
+    if (!xyz && !(a < 2 && xy)) h->tile[a] = h->tuned[a];
   invalidate_graph(h);
   if (shape_out)
     for (int a = 0; a < 3; a++) shape_out[a] = h->tile[a];

@@ -325,7 +325,8 @@ class Block(BlockBase):
 
     def autotune(self, reps=5):
         """Time every tile shape of each axis' sweep on the current state and
-        keep the fastest; returns the chosen shapes.  Overwrites du."""
+        keep the fastest; returns the chosen shapes (0 for axes that run
+        together in one launch).  Overwrites du."""
         a = (ctypes.c_int32 * 3)()
         self._call("autotune", ctypes.c_int32(reps), a)
         return list(a)
