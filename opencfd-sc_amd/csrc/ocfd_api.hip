@@ -50,9 +50,24 @@ struct ProfRec {
 // characteristic 96^3 1172 and 1180, 104^3 1565 and 1611; hybrid 96^3 1728 and
 // 1733, 112^3 2077 and 2151; WENO5 characteristic plate 200 x 100 x 40 1608 and
 // 1610.
+// One launch runs one instance for the three axes, so beside an axis that
+// closes, or is askew, the projecting schemes' other two run without the
+// reduced basis of an aligned metric vector.  In FP64 that costs more than the
+// launches from some 3 10^5 cells on.  One closed axis, three launches with
+// tuned and default tiles, and one: WENO7 characteristic 48^3 353, 361 and 327,
+// 64^3 498, 498 and 486, 80^3 920, 974 and 953, 120 x 100 x 48 932, 976 and 1011;
+// WENO5 characteristic 64^3 405, 405 and 403, 80^3 742, 773 and 776, 120 x 100 x
+// 48 732, 765 and 806.  Mixed precision, WENO7 characteristic 80^3 522, 547 and
+// 505; with a single aligned axis FP64 80^3 1112, 1116 and 1085.
 // (The mass force is added by the z sweep.)
-constexpr int64_t XYZ_MAX_CELLS = 600000;
-bool xyz_wins(const Block &B) { return B.P.if_mass_force != 1 && B.g.ni <= XYZ_MAX_CELLS; }
+constexpr int64_t XYZ_MAX_CELLS = 600000, XYZ_MAX_CELLS_MIXED_AXES = 300000;
+bool xyz_wins(const Block &B) {
+  if (B.P.if_mass_force == 1) return false;
+  const bool basis = B.S.is_char && B.S.scheme_invis != SCH_HYBRID && B.M.uniform && B.prec == OCFD_PREC_FP64_CODE;
+  const int reduced = (B.S.iperiodic[0] == 1 && axis_aligned<0>(B.M)) + (B.S.iperiodic[1] == 1 && axis_aligned<1>(B.M)) +
+                      (B.S.iperiodic[2] == 1 && axis_aligned<2>(B.M));
+  return B.g.ni <= (basis && reduced == 2 ? XYZ_MAX_CELLS_MIXED_AXES : XYZ_MAX_CELLS);
+}
 }  // namespace
 
 struct ocfd_handle {
