@@ -482,12 +482,18 @@ int inviscid(ocfd_handle *h, bool ch, bool xyz = false) {
   return 0;
 }
 
+// ocfd_handle::pend bits (stage fusion)
+constexpr int PEND_VISC = 1, PEND_UPDATE = 2, PEND_REFRESHED = 4, PEND_UVW = 8, PEND_HALO = 16;
+
 // the halo fill at the start of a whole step's stage
 int exchange_stage(ocfd_handle *h) {
   return launch(h, "halo_fill", [&] { return launch_halo_both(h->B, h->st); });
 }
 
 int exchange_prims(ocfd_handle *h) {
+  // one buffer of T and set of u, v, w only: inside a fused stage its repair
+  // copies the halos again
+  h->pend &= ~PEND_HALO;
   const PrimField f[5] = {h->B.d, h->B.u, h->B.v, h->B.w, h->B.T};
   return launch(h, "halo_fill", [&] { return launch_halo_prims(h->B, f, 5, h->st); });
 }
@@ -562,9 +568,6 @@ void swap_uvw(ocfd_handle *h) {
   std::swap(h->B.w, h->B.w2);
   h->uvpar ^= 1;
 }
-
-// ocfd_handle::pend bits (stage fusion)
-constexpr int PEND_VISC = 1, PEND_UPDATE = 2, PEND_REFRESHED = 4, PEND_UVW = 8, PEND_HALO = 16;
 
 int read_neg(ocfd_handle *h, int out[3]) {
   HIPCHK(hipMemcpyAsync(out, h->neg, sizeof(int), hipMemcpyDeviceToHost, h->st));
@@ -968,7 +971,7 @@ int ocfd_get_time(ocfd_handle *h, int32_t *istep, double *tt) {
 
 // ---- one reference routine each ---------------------------------------------
 int ocfd_exchange_primitives(ocfd_handle *h) {
-  if (h->stage_fusion && h->halo_both) {
+  if (h->stage_fusion && h->halo_both && !(h->pend & PEND_UPDATE)) {
     h->pend |= PEND_HALO;
     return exchange_stage(h);
   }
@@ -1445,6 +1448,7 @@ int ocfd_show_flow_msg_noalloc(ocfd_handle *h, double out[3]) {
 
 int ocfd_ana_box(ocfd_handle *h, double out[20]) {
   const PrimField uvw[3] = {h->B.u, h->B.v, h->B.w};
+  h->pend &= ~PEND_HALO;  // one set of u, v, w (exchange_prims)
   if (launch(h, "halo_fill", [&] { return launch_halo_prims(h->B, uvw, 3, h->st); })) return -1;
   if (launch(h, "ana_box", [&] { return launch_ana_box(h->B, nullptr, nullptr, h->work, h->wout, h->st); }))
     return -1;
