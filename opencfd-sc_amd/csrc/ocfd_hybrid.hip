@@ -17,6 +17,7 @@
 // same expression as in the sweep (flux_charteric,
 // OCFD_inviscous_character.f90:190-290; OCFD2d_flux1/2,
 // OCFD_inviscous.f90:210-361), so results are unchanged bit for bit.
+#include <algorithm>
 #include <type_traits>
 
 #include "ocfd_kernels.h"
@@ -403,31 +404,17 @@ __global__ __launch_bounds__(WNT) void k_weno_faces(const Block B, const int nwg
   else weno_faces_axis<2, CHAR, MET, RR>(B, sF, sQ, sG, wg, nwg);
 }
 
-// As many workgroups per axis as the device holds at once (CUs x resident
-// workgroups per CU), so that the batches spread evenly, and no more than the
-// axis can have batches.
-template <typename K>
-int weno_groups(K kernel, int64_t faces, int (&cache)[64]) {
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (cache[dev] == 0) {
-    int cus = 0, per = 0;
-    if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, WNT, 0) != hipSuccess || per < 1) per = 1;
-    cache[dev] = cus * per;
-  }
-  const int64_t most = ((faces + NSUB * FB - 1) / (NSUB * FB) + NXCD - 1) / NXCD * NXCD;
-  return (int)(most < cache[dev] ? most : cache[dev]);
-}
-
 template <int AXIS, bool CHAR, int MET, typename RR>
 hipError_t weno_launch(const Block &B, hipStream_t st) {
-  static int cache[64] = {};
+  static DeviceCache cache;
   const Geom &g = B.g;
   int64_t faces = TileIndex<0>::nfaces(g);
   if (AXIS != 0 && TileIndex<1>::nfaces(g) > faces) faces = TileIndex<1>::nfaces(g);
   if (AXIS != 0 && TileIndex<2>::nfaces(g) > faces) faces = TileIndex<2>::nfaces(g);
-  const int nwg = weno_groups(k_weno_faces<AXIS, CHAR, MET, RR>, faces, cache);
+  // as many workgroups per axis as the device holds at once, so that the batches
+  // spread evenly, and no more than the axis can have batches
+  const int64_t most = ((faces + NSUB * FB - 1) / (NSUB * FB) + NXCD - 1) / NXCD * NXCD;
+  const int nwg = (int)std::min<int64_t>(most, resident_groups(k_weno_faces<AXIS, CHAR, MET, RR>, cache, WNT));
   hipLaunchKernelGGL((k_weno_faces<AXIS, CHAR, MET, RR>), dim3((unsigned)(AXIS >= 0 ? nwg : 3 * nwg)), dim3(WNT), 0,
                      st, B, nwg);
   return hipGetLastError();

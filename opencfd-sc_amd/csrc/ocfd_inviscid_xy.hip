@@ -302,7 +302,7 @@ void k_inviscid_xy(const Block B, const int sl) {
 // shortest segments (FP64 256^3: 7 segments 600 us, 5 639).
 template <typename R, bool SW>
 int xy_segment(const Geom &g, int64_t &work) {
-  static int cache[64] = {};
+  static DeviceCache cache;
   const int64_t slots = resident_groups(k_inviscid_xy<R, SW>, cache, XYW);
   const int64_t cols = (int64_t)((g.nx + XYW - 1) / XYW) * g.nz;
   int best = 0;

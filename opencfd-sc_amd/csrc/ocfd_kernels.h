@@ -2,6 +2,7 @@
 // gfx950 kernels (definitions in the .hip files of this directory).
 #pragma once
 #include "ocfd_common.h"
+#include "ocfd_device_cache.h"
 
 namespace ocfd {
 
@@ -390,16 +391,15 @@ constexpr int NT = 256;
 // workgroups of `kernel` (static LDS) the device holds at once;
 // `cache` keeps the value per device for one kernel
 template <typename K>
-int resident_groups(K kernel, int (&cache)[64], int threads = NT) {
+int resident_groups(K kernel, DeviceCache &cache, int threads = NT) {
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) dev = 0;
-  if (cache[dev] == 0) {
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= DeviceCache::DEVICES) dev = 0;
+  return cache.get(dev, [&] {
     int cus = 0, per = 0;
     if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || cus < 1) cus = 256;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per, kernel, threads, 0) != hipSuccess || per < 1) per = 1;
-    cache[dev] = cus * per;
-  }
-  return cache[dev];
+    return cus * per;
+  });
 }
 
 // interior (i, j, k), 1-based, of cell t of the nx * ny * nz block (i fastest)

@@ -610,7 +610,7 @@ inline bool all_periodic(const Block &B) {
 
 template <bool CD8, bool FAST, typename RT>
 void launch_flux_one(const Block &B, hipStream_t st) {
-  static int cache[64] = {};
+  static DeviceCache cache;
   const int kseg = march_kseg(B.g, resident_groups(k_visc_flux<CD8, FAST, RT>, cache), march_kmax<RT>());
   hipLaunchKernelGGL((k_visc_flux<CD8, FAST, RT>), dim3(march_blocks(B.g, kseg)), dim3(NT), 0, st, B, kseg);
 }
@@ -632,7 +632,7 @@ hipError_t visc_div_as(const Block &B, hipStream_t st) {
 
 template <bool VISC, bool CD8, bool FAST, typename RT, bool TRI>
 void launch_update_one(const Block &B, int krk, int refresh_planes, int *neg, hipStream_t st) {
-  static int cache[64] = {};
+  static DeviceCache cache;
   const int kseg =
       march_kseg(B.g, resident_groups(k_visc_div_update<VISC, CD8, FAST, RT, TRI>, cache), march_kmax<RT>());
   hipLaunchKernelGGL((k_visc_div_update<VISC, CD8, FAST, RT, TRI>), dim3(march_blocks(B.g, kseg)), dim3(NT), 0, st, B,

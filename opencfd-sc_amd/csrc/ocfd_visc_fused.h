@@ -375,7 +375,7 @@ hipError_t visc_fused_batch_as(const BoxSet &S, int krk, int *neg, int ntiles, h
 
 template <typename RT, bool TRI>
 void visc_fused_one(const Block &B, int krk, int refresh, int *neg, hipStream_t st) {
-  static int cache[64] = {};
+  static DeviceCache cache;
   const int kseg = fused_kseg(B.g, resident_groups(k_visc_fused<RT, TRI>, cache));
   hipLaunchKernelGGL((k_visc_fused<RT, TRI>), dim3(fused_blocks(B.g, kseg)), dim3(NT), 0, st, B, krk, refresh, kseg, neg);
 }
