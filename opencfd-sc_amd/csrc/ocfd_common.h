@@ -125,9 +125,12 @@ __device__ inline float maddx(float a, float b, float k, float c) { return __bui
 // quotient by the steps of the compiler's division (reciprocal, two Newton
 // iterations, quotient and remainder correction, v_div_fixup for zeros,
 // infinities and NaN) without its two v_div_scale, which leave operands
-// alone whose exponents are far from the ends of the range: the weights'
-// denominators (ep + S)^2 are at least 1e-16, and the results are the same
-// bits while no flux exceeds 1e76 and no numerator lies below 1e-292.
+// alone whose exponents are far from the ends of the range.  Results are the
+// same bits while the denominator (ep + S)^2, at least 1e-16, is below 2^1016
+// -- the square itself overflows from 2^1024 on, at fluxes 4 times larger, some
+// 1e76 -- and no numerator but 0 lies below 1e-292, i.e. no reconstructed flux
+// but 0 below some 1e-304.  (With the general division WENO7 characteristic
+// steps of 192^3 and WENO5 characteristic plates take 2% longer.)
 // FP32: a product with the hardware reciprocal (within 1 ulp), which stays
 // far inside the mixed form's accuracy, set by its FP32 fluxes.
 __device__ inline double wdiv(double a, double b) {
