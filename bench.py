@@ -541,12 +541,17 @@ def cpu_baseline(workload: str, mode: str):
 
 
 # ---------------------------------------------------------------------------
-def tiles_desc(b):
+def tiles_desc(b, prof):
     """Sweep launch shapes per axis: tiles (points x lines) or y/z marches
-    (one lane per line, segments of 32 or 64 cells)."""
+    (one lane per line, segments of 32 or 64 cells); axes that the profiled
+    steps swept together as such."""
     out = []
     for a, s in enumerate(b.tiles):
-        if s >= 3:
+        if "inviscid_xyz" in prof:
+            out.append("one launch")
+        elif a < 2 and "inviscid_char_xy" in prof:
+            out.append("x+y march")
+        elif s >= 3:
             out.append("march%d" % (32 if s == 3 else 64))
         else:
             tl = (64, 32, 128)[s] if a == 0 else (32, 16, 64)[s]
@@ -635,7 +640,7 @@ def main():
         if r["mix"]:
             out["face_mix_linear_weno7_weno5"] = [round(x, 5) for x in r["mix"]]
         if args.autotune:
-            out["sweep_tiles_xyz"] = tiles_desc(r["b"])
+            out["sweep_tiles_xyz"] = tiles_desc(r["b"], r["prof"])
         return out
 
     main_r = runs[prec]
