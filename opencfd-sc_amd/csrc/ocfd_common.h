@@ -407,8 +407,9 @@ __device__ inline T omp6_core(T xm3, T xm2, T xm1, T x0, T x1, T x2,
   constexpr T kappa = T(4.0);
   // Products with 2, 4 and 0.5 are exact, so their sums are fused (xmadd); a
   // stencil with a NaN makes mid a NaN, which skips the limiter.  The limiter
-  // is 54 FP64 instructions instead of 190 and runs for nearly every
-  // wavefront: OMP6 sweeps of 128^3 FP64 92-124 us per launch before, 63-79 now.
+  // is 55 FP64 instructions (of 82 in all) instead of 190 and runs for nearly
+  // every wavefront: OMP6 sweeps of 128^3 FP64 133-138 us per launch before all
+  // changes of the sweeps, 81-84 now.
   T mid = a1 * x4 + a2 * x3 + a3 * x2 + a4 * x1 + a5 * x0 + a6 * xm1 + a7 * xm2 + a8 * xm3;
   const T dl = x0 - xm1, dr = x1 - x0;
   const T mp = x0 + minmod2(dr, kappa * dl);

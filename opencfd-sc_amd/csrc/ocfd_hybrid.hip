@@ -105,8 +105,8 @@ __device__ __forceinline__ void hyb_list_axis(const Block &B, int (&soff)[LPT][N
 }
 
 // the lists of the three axes: workgroups [0, n0) x, [n0, n0 + n1) y, then z
-// (256^3 184 us in three launches with one face's loads at a time, 155 now;
-// 101 x 75 x 54 35 and 11.5)
+// (256^3 181 us in three launches with one face's loads at a time, 147 now;
+// 101 x 75 x 54 34 and 11)
 __global__ __launch_bounds__(NT) void k_hyb_list(const Block B, const unsigned n0, const unsigned n1) {
   __shared__ int soff[LPT][NT / 64];
   __shared__ int sbase;
@@ -139,12 +139,12 @@ using weno_lds_t = typename std::conditional<CHAR, double, RR>::type;
 // as the arithmetic of a batch), and a lane keeps its face's coefficients in
 // registers to the end: two barriers per batch.  A workgroup takes three
 // batches at once: as workgroups of five wavefronts only two fitted a CU (the
-// first SIMD takes two of each five), 2.1 wavefronts per SIMD instead of 3.7.
-// Bound by instruction issue (VALU 65% busy).  256^3, 5.7% of the faces, three
-// axes: FP64 780 us in the former layout (256 lanes on 51 faces, one lane per
-// row: every lane formed all rows' entries, three launches), 695 with five
-// wavefronts per workgroup, 527 now; mixed (8.3%) 705, 550, 516; 160^3 FP64
-// with metric fields (8.6%) 414, 372, 305.
+// first SIMD takes two of each five), 2.1 wavefronts per SIMD instead of 3.7,
+// which was half of the gain.  Bound by instruction issue (VALU 65% busy).  The
+// three axes in the former layout (256 lanes on 51 faces, one lane per row:
+// every lane formed all rows' entries, three launches) and now: 256^3 FP64,
+// 3.9% of the faces listed, 609 and 406 us; mixed (5.7%) 389 and 275; 160^3
+// FP64 with metric fields (10%) 428 and 306; 101 x 75 x 54 mixed (28%) 49 and 38.
 template <int AXIS, bool CHAR, int MET, typename RR>
 __device__ __forceinline__ void weno_faces_axis(const Block &B, weno_lds_t<CHAR, RR> *const sFa, double *const sQa,
                                                 double *const sGa,

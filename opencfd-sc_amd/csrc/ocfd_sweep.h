@@ -298,8 +298,8 @@ __device__ __forceinline__ void sweep_tile(const Block &B, int b, const int mode
   // others stays, so finite fluxes are the same bits.  The projection of
   // two rows and 96 of 400 LDS reads per face go, and the rows' code is
   // straight-line (the loop of face_ch indexes its row at run time).  WENO7
-  // sweeps of 192^3: FP64 835-857 us with the general form, 650-710 with this
-  // one; FP32 330-355 and 270-293.
+  // sweeps of 192^3, default tiles: FP64 765-774 us with the general form,
+  // 645-693 with this one; FP32 306-316 and 278-297.
   auto face_aligned = [&](int f, int wl, R *hh) {
     FACE_STENCIL;
     constexpr int IL = AXIS == 0 ? 1 : 0, IM = AXIS == 2 ? 1 : 2;  // the tangents' coordinates
