@@ -111,10 +111,11 @@ struct ocfd_handle {
   // and the repair copies none (mixed 256^3: repair 61 -> 4 us per stage)
   bool halo_both = false;
   // small blocks: the y and z parts of du of whole steps, whose three sweeps
-  // are one launch (k_inviscid_xyz), in the sweeps' real type; allocated by the
-  // first whole step (ensure_parts), NULL where the sweeps run one by one
+  // are one launch (k_inviscid_xyz), in the sweeps' real type; allocated when
+  // the block gets its state (ensure_parts), NULL where the sweeps run one by one
   char *du_yz = nullptr;
   bool parts_tried = false;
+  bool in_batch = false;  // a box of an ocfd_batch
   // whole steps take the three sweeps in one launch, once there is room
   bool joins_xyz() const { return !tile[0] && !tile[1] && !tile[2] && (du_yz || !parts_tried) && xyz_wins(B); }
   bool joined_xyz() const { return du_yz && joins_xyz(); }
@@ -378,6 +379,25 @@ int prim_upload(ocfd_handle *h, int q, const double *src) {
   return 0;
 }
 
+// Room for the parts, when the block gets its state: after every array it cannot
+// do without, and not inside the first step (64^3 with metric fields, a first
+// pass of 10 steps: 4.27 ms with the allocation, 3.54 without).  Boxes of a
+// batch, whose sweeps run one by one, take it when they first step alone.
+// Without room the sweeps run one by one.
+int ensure_parts(ocfd_handle *h) {
+  if (h->parts_tried || !h->joins_xyz()) return 0;
+  h->parts_tried = true;
+  int cur = 0;
+  HIPCHK(hipGetDevice(&cur));
+  if (cur != h->device) HIPCHK(hipSetDevice(h->device));
+  if (hipMalloc((void **)&h->du_yz, 2 * h->part_bytes()) != hipSuccess) {
+    h->du_yz = nullptr;
+    (void)hipGetLastError();
+  }
+  if (cur != h->device) HIPCHK(hipSetDevice(cur));
+  return 0;
+}
+
 // the second buffers of T and u, v, w hold the halos (edges and corners
 // included) of the first after an upload (ocfd_handle::halo_both)
 int copy_second(ocfd_handle *h) {
@@ -407,7 +427,7 @@ int upload_prims(ocfd_handle *h, const double *const src[5], bool make_f) {
     if (make_f && launch(h, "init_f", [&] { return launch_init_f(h->B, h->st); })) return -1;
     if (copy_second(h)) return -1;
     HIPCHK(hipStreamSynchronize(h->st));
-    return 0;
+    return h->in_batch ? 0 : ensure_parts(h);
   }
   int rc = 0;
   if (make_f) {
@@ -426,6 +446,7 @@ int upload_prims(ocfd_handle *h, const double *const src[5], bool make_f) {
   }
   for (int q = 0; q < 5 && !rc; q++) rc = prim_upload(h, q, src[q]);
   if (!rc) rc = copy_second(h);
+  if (!rc && !h->in_batch) rc = ensure_parts(h);
   return rc;
 }
 
@@ -434,22 +455,6 @@ Block with_parts(const ocfd_handle *h, Block B) {
   B.du2 = reinterpret_cast<double *>(h->du_yz);
   B.du3 = reinterpret_cast<double *>(h->du_yz + h->part_bytes());
   return B;
-}
-// Room for the parts, on the first whole step: the boxes of a batch, whose
-// sweeps run one by one, and blocks driven by the routines never need it, and
-// every block's own arrays come first.  Without room the sweeps run one by one.
-int ensure_parts(ocfd_handle *h) {
-  if (h->parts_tried || !h->joins_xyz()) return 0;
-  h->parts_tried = true;
-  int cur = 0;
-  HIPCHK(hipGetDevice(&cur));
-  if (cur != h->device) HIPCHK(hipSetDevice(h->device));
-  if (hipMalloc((void **)&h->du_yz, 2 * h->part_bytes()) != hipSuccess) {
-    h->du_yz = nullptr;
-    (void)hipGetLastError();
-  }
-  if (cur != h->device) HIPCHK(hipSetDevice(cur));
-  return 0;
 }
 // du as the z sweep leaves it, for its readers outside whole steps
 int settle_du(ocfd_handle *h) {
@@ -1846,6 +1851,7 @@ int ocfd_batch_create(const ocfd_config *cfgs, int32_t nbox, int32_t device, ocf
       batch_free(b);
       return fail(msg);
     }
+    h->in_batch = true;
     b->box.push_back(h);
     b->cells += (int64_t)cfgs[i].nx * cfgs[i].ny * cfgs[i].nz;
   }

@@ -2,6 +2,7 @@
 y and z parts of the right-hand side belong to whole steps of a box alone)."""
 import ctypes
 
+import numpy as np
 import pytest
 
 from ocfd import cases, native
@@ -39,3 +40,22 @@ def test_batch_footprint(precision):
         assert "inviscid_xyz" in box.profile_read()
         parts = 10 * plane * (4 if precision else 8)
         assert before1 - _free() <= parts * 1.1 + (16 << 20)
+
+
+@pytest.mark.parametrize("precision", [0, 1])
+def test_first_step_of_a_block_allocates_nothing_large(precision):
+    """A block alone takes the parts with its state, not inside its first step."""
+    n = 80
+    case = cases.random_case(shape=(16, 16, 32), seed=85)
+    cfg = case.cfg.replace(nx=n, ny=n, nz=n, metric_mode=1, precision=precision)
+    with native.Block(cfg) as b:
+        b.set_uniform_metrics(cases.uniform_box_metrics(n, n, n))
+        b.upload_primitives([np.ones(cfg.halo_shape)] * 5)
+        b.bc()
+        b.synchronize()
+        before = _free()
+        b.step(1)
+        assert before - _free() < 10 * n ** 3 * (4 if precision else 8) // 2
+        b.profile_enable(True)
+        b.step(1)
+        assert "inviscid_xyz" in b.profile_read()
