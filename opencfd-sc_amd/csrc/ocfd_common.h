@@ -149,7 +149,9 @@ __device__ inline float ediv(float a, float b) { return a / b; }
 // quotient and one remainder correction give the correctly rounded a / b
 // (Markstein; Brisebarre, Muller and Raina, "Accelerating correctly rounded
 // floating-point division when the divisor is known in advance", 2004), in 3
-// instructions instead of the general division's 11
+// instructions instead of the general division's 11.  (Where the remainder
+// underflows, below some 1e-292 in FP64, the last bit may differ; an infinite a
+// gives NaN.)
 __device__ inline double div_known(double a, double b, double rb) {
   const double q = a * rb;
   return __builtin_fma(__builtin_fma(-b, q, a), rb, q);
